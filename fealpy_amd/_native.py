@@ -41,6 +41,8 @@ _SIGNATURES = {
     "fa_element_vectors": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p, _i64,
                                           _p, _p, ctypes.c_int, _f64, _p, _p, _p]),
     "fa_gather_matrix": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _p, _p]),
+    "fa_row_positions": (ctypes.c_int, [_i64, _i32, _p, _p, _p, _p, _p, _i32, _p, _p]),
+    "fa_sum_rows": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _i32, _p, _i64, _p, _p]),
     "fa_gather_vector": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _p]),
     "fa_element_apply": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _i64, _p, _p, _p]),
     "fa_element_elasticity": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p, _i64, _p,
@@ -105,6 +107,7 @@ _SIGNATURES = {
     "fa_p1_box_matrix": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p, ctypes.c_int,
                                         _p, _p, ctypes.c_int, _f64, _p, ctypes.c_int, _f64, _p, _p, _i64, _p, _p]),
     "fa_sep_points": (ctypes.c_int, [_p, ctypes.c_int64, ctypes.c_int, _p, _p, _p]),
+    "fa_sep_sample": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _p, _p, _i64, _p, _p, _p]),
     "fa_box_axes_work_bytes": (_sz, []),
     "fa_box_axes": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p, _p, _p, _sz, _p]),
     "fa_p1_box_vector_work_bytes": (_sz, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),

@@ -8,65 +8,6 @@
 
 namespace fa {
 
-// One thread per (cell, row i); the row of the element matrix is kept in
-// registers (LDOF is a compile-time constant).
-template <int TD, int LDOF, class T, bool SEP>
-__global__ void __launch_bounds__(256) k_element_matrices(const double* __restrict__ node, const int32_t* __restrict__ cell,
-                                                         int64_t nc, int nq, const double* __restrict__ qw,
-                                                         const double* __restrict__ phi, const double* __restrict__ gphi,
-                                                         int dk, double ds, const double* __restrict__ dc, int mk,
-                                                         double ms, const double* __restrict__ mc, T* __restrict__ elem) {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= nc * LDOF) return;
-    const int64_t c = t / LDOF;
-    const int i = static_cast<int>(t - c * LDOF);
-    double p[TD + 1][TD];
-    load_cell<TD>(node, cell, c, p);
-    Geom<TD> g;
-    g.compute(p);
-    double acc[LDOF];
-#pragma unroll
-    for (int j = 0; j < LDOF; ++j) acc[j] = 0.0;
-    for (int q = 0; q < nq; ++q) {
-        const double wq = qw[q] * g.meas;
-        if (dk) {
-            const double kd = wq * coef_at<TD, SEP>(dk, ds, dc, c, c, q, nq, p);
-            const double* R = gphi + (int64_t)q * LDOF * (TD + 1);
-            double gi[TD];
-#pragma unroll
-            for (int d = 0; d < TD; ++d) {
-                double s = 0.0;
-#pragma unroll
-                for (int a = 0; a < TD + 1; ++a) s += R[i * (TD + 1) + a] * g.gl[a][d];
-                gi[d] = s;
-            }
-#pragma unroll
-            for (int j = 0; j < LDOF; ++j) {
-                double dot = 0.0;
-#pragma unroll
-                for (int d = 0; d < TD; ++d) {
-                    double s = 0.0;
-#pragma unroll
-                    for (int a = 0; a < TD + 1; ++a) s += R[j * (TD + 1) + a] * g.gl[a][d];
-                    dot += gi[d] * s;
-                }
-                acc[j] += kd * dot;
-            }
-        }
-        if (mk) {
-            const double km = wq * coef_at<TD, SEP>(mk, ms, mc, c, c, q, nq, p);
-            const double* ph = phi + (int64_t)q * LDOF;
-            const double pi = ph[i] * km;
-#pragma unroll
-            for (int j = 0; j < LDOF; ++j) acc[j] += pi * ph[j];
-        }
-    }
-    T* out = elem + t * LDOF;
-#pragma unroll
-    for (int j = 0; j < LDOF; ++j) out[j] = static_cast<T>(acc[j]);
-}
-
-// ---- fixed-order gather ---------------------------------------------------
 __device__ inline int lower_bound_lds(const int32_t* a, int n, int32_t v) {
     int lo = 0, hi = n;
     while (lo < hi) {
@@ -75,85 +16,6 @@ __device__ inline int lower_bound_lds(const int32_t* a, int n, int32_t v) {
         else hi = mid;
     }
     return lo;
-}
-
-// G lanes per global row (G >= ldof); each row's columns and accumulators
-// live in LDS.  The incident cells of a row are visited in ascending order
-// and lane j adds element entry (i, j) of the current cell, so every CSR entry
-// is summed in ascending cell order -- the order of the reference's stable
-// lexsort + sequential np.add.at.  Distinct columns of one cell never collide.
-template <class T, int G>
-__global__ void k_gather_matrix(int64_t gdof, int ldof, const int32_t* __restrict__ c2d,
-                                const int32_t* __restrict__ ptr, const int32_t* __restrict__ adj,
-                                const int32_t* __restrict__ indptr, const int32_t* __restrict__ indices, int lmax,
-                                const T* __restrict__ elem, int64_t cstride, T* __restrict__ values) {
-    extern __shared__ char smem[];
-    const int rpb = blockDim.x / G;
-    const int sub = threadIdx.x / G;
-    const int lane = threadIdx.x % G;
-    int32_t* cols = reinterpret_cast<int32_t*>(smem) + sub * lmax;
-    T* acc = reinterpret_cast<T*>(smem + align_up(sizeof(int32_t) * rpb * lmax, 16)) + sub * lmax;
-    for (int64_t r = (int64_t)blockIdx.x * rpb + sub; r < gdof; r += (int64_t)gridDim.x * rpb) {
-        const int32_t r0 = indptr[r];
-        const int L = indptr[r + 1] - r0;
-        for (int t = lane; t < L; t += G) {
-            cols[t] = indices[r0 + t];
-            acc[t] = T(0);
-        }
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-        const int32_t k1 = ptr[r + 1];
-        if (ldof <= G) {
-            // the row's incidences G at a time in one load, handed out by
-            // shuffles; the next incidence's column and value loads are issued
-            // before the current one's search and add (same adds, same order)
-            for (int32_t kb = ptr[r]; kb < k1; kb += G) {
-                const int32_t mine = kb + lane < k1 ? adj[kb + lane] : 0;
-                const int nk = min(G, k1 - kb);
-                const bool act = lane < ldof;
-                int32_t e = __shfl(mine, 0, G);
-                int32_t c = e / ldof;
-                int32_t col = act ? c2d[(int64_t)c * ldof + lane] : 0;
-                T v = act ? elem[(int64_t)c * cstride + (e - c * ldof) * ldof + lane] : T(0);
-                for (int u = 0; u < nk; ++u) {
-                    int32_t col_n = 0;
-                    T v_n = T(0);
-                    if (u + 1 < nk) {
-                        const int32_t en = __shfl(mine, u + 1, G);
-                        const int32_t cn = en / ldof;
-                        if (act) {
-                            col_n = c2d[(int64_t)cn * ldof + lane];
-                            v_n = elem[(int64_t)cn * cstride + (en - cn * ldof) * ldof + lane];
-                        }
-                    }
-                    if (act) {
-                        const int pos = lower_bound_lds(cols, L, col);
-                        if (pos < L && cols[pos] == col) acc[pos] += v;
-                    }
-                    __builtin_amdgcn_wave_barrier();
-                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-                    col = col_n;
-                    v = v_n;
-                }
-            }
-        } else {
-            for (int32_t k = ptr[r]; k < k1; ++k) {
-                const int32_t e = adj[k];
-                const int32_t c = e / ldof;
-                for (int j = lane; j < ldof; j += G) {
-                    const int32_t col = c2d[(int64_t)c * ldof + j];
-                    const T v = elem[(int64_t)c * cstride + (e - c * ldof) * ldof + j];
-                    const int pos = lower_bound_lds(cols, L, col);
-                    if (pos < L && cols[pos] == col) acc[pos] += v;
-                }
-                __builtin_amdgcn_wave_barrier();
-                __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-            }
-        }
-        for (int t = lane; t < L; t += G) values[r0 + t] = acc[t];
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    }
 }
 
 // physical coordinates of barycentric points on every cell: one thread per
@@ -569,104 +431,9 @@ static int launch_p1(int64_t gdof, const double* node, const int32_t* cell, int 
     return FA_OK;
 }
 
-template <int TD, int LDOF, class T>
-static void launch_elem(const double* node, const int32_t* cell, int64_t nc, int nq, const double* qw,
-                        const double* phi, const double* gphi, int dk, double ds, const double* dc, int mk, double ms,
-                        const double* mc, void* elem, hipStream_t s) {
-    const int64_t n = nc * LDOF;
-    if (dk == FA_COEF_SEP || mk == FA_COEF_SEP)
-        hipLaunchKernelGGL((k_element_matrices<TD, LDOF, T, true>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           node, cell, nc, nq, qw, phi, gphi, dk, ds, dc, mk, ms, mc, static_cast<T*>(elem));
-    else
-        hipLaunchKernelGGL((k_element_matrices<TD, LDOF, T, false>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s,
-                           node, cell, nc, nq, qw, phi, gphi, dk, ds, dc, mk, ms, mc, static_cast<T*>(elem));
-}
-
-template <class T>
-static int dispatch_elem(int td, int ldof, const double* node, const int32_t* cell, int64_t nc, int nq,
-                         const double* qw, const double* phi, const double* gphi, int dk, double ds, const double* dc,
-                         int mk, double ms, const double* mc, void* elem, hipStream_t s) {
-#define FA_ELEM_CASE(TD_, L_)                                                                             \
-    if (td == TD_ && ldof == L_) {                                                                        \
-        launch_elem<TD_, L_, T>(node, cell, nc, nq, qw, phi, gphi, dk, ds, dc, mk, ms, mc, elem, s);      \
-        FA_LAUNCH("k_element_matrices");                                                                  \
-        return FA_OK;                                                                                     \
-    }
-    FA_ELEM_CASE(2, 3) FA_ELEM_CASE(2, 6) FA_ELEM_CASE(2, 10) FA_ELEM_CASE(2, 15)
-    FA_ELEM_CASE(3, 4) FA_ELEM_CASE(3, 10) FA_ELEM_CASE(3, 20) FA_ELEM_CASE(3, 35)
-#undef FA_ELEM_CASE
-    set_error("fa_element_matrices: unsupported (td=%d, ldof=%d); p must be 1..4", td, ldof);
-    return FA_EINVAL;
-}
-
-template <class T, int G>
-static int launch_gather(int64_t gdof, int ldof, const int32_t* c2d, const int32_t* ptr, const int32_t* adj,
-                         const int32_t* indptr, const int32_t* indices, int lmax, const void* elem, int64_t cstride,
-                         void* values, hipStream_t s) {
-    const size_t per_row = sizeof(int32_t) * lmax + sizeof(T) * lmax;
-    int rpb = 256 / G;
-    while (rpb > 1 && rpb * per_row + 16 > 48 * 1024) rpb >>= 1;
-    const size_t lds = align_up(sizeof(int32_t) * rpb * lmax, 16) + sizeof(T) * rpb * lmax;
-    if (lds > 64 * 1024) {
-        set_error("fa_gather_matrix: row length %d exceeds the LDS capacity", lmax);
-        return FA_ECAPACITY;
-    }
-    const unsigned grid = grid_for(gdof, rpb, 1 << 20);
-    hipLaunchKernelGGL((k_gather_matrix<T, G>), dim3(grid), dim3(rpb * G), lds, s, gdof, ldof, c2d, ptr, adj, indptr,
-                       indices, lmax, static_cast<const T*>(elem), cstride, static_cast<T*>(values));
-    FA_LAUNCH("k_gather_matrix");
-    return FA_OK;
-}
-
-template <class T>
-static int dispatch_gather(int64_t gdof, int ldof, const int32_t* c2d, const int32_t* ptr, const int32_t* adj,
-                           const int32_t* indptr, const int32_t* indices, int lmax, const void* elem, int64_t cs,
-                           void* values, hipStream_t s) {
-    if (ldof <= 4) return launch_gather<T, 4>(gdof, ldof, c2d, ptr, adj, indptr, indices, lmax, elem, cs, values, s);
-    if (ldof <= 8) return launch_gather<T, 8>(gdof, ldof, c2d, ptr, adj, indptr, indices, lmax, elem, cs, values, s);
-    if (ldof <= 16)
-        return launch_gather<T, 16>(gdof, ldof, c2d, ptr, adj, indptr, indices, lmax, elem, cs, values, s);
-    if (ldof <= 32)
-        return launch_gather<T, 32>(gdof, ldof, c2d, ptr, adj, indptr, indices, lmax, elem, cs, values, s);
-    return launch_gather<T, 64>(gdof, ldof, c2d, ptr, adj, indptr, indices, lmax, elem, cs, values, s);
-}
-
 }  // namespace fa
 
 using namespace fa;
-
-extern "C" int fa_element_matrices(int dtype, int td, int ldof, int nq, const double* node, const int32_t* cell,
-                                   int64_t nc, const double* qw, const double* phi, const double* gphi_u,
-                                   int diff_kind, double diff_scale, const double* diff_coef, int mass_kind,
-                                   double mass_scale, const double* mass_coef, void* elem, fa_stream_t stream) {
-    FA_REQUIRE(dtype == FA_F64 || dtype == FA_F32, "fa_element_matrices: bad dtype %d", dtype);
-    FA_REQUIRE(nq > 0 && nc >= 0, "fa_element_matrices: bad sizes");
-    FA_REQUIRE(!diff_kind || gphi_u, "fa_element_matrices: diffusion needs gphi_u");
-    FA_REQUIRE(!mass_kind || phi, "fa_element_matrices: mass needs phi");
-    FA_REQUIRE(!(diff_kind >= FA_COEF_CELL && !diff_coef) && !(mass_kind >= FA_COEF_CELL && !mass_coef),
-               "fa_element_matrices: coefficient array missing");
-    if (nc == 0) return FA_OK;
-    if (dtype == FA_F64)
-        return dispatch_elem<double>(td, ldof, node, cell, nc, nq, qw, phi, gphi_u, diff_kind, diff_scale, diff_coef,
-                                     mass_kind, mass_scale, mass_coef, elem, S(stream));
-    return dispatch_elem<float>(td, ldof, node, cell, nc, nq, qw, phi, gphi_u, diff_kind, diff_scale, diff_coef,
-                                mass_kind, mass_scale, mass_coef, elem, S(stream));
-}
-
-extern "C" int fa_gather_matrix(int dtype, int64_t gdof, int32_t ldof, const int32_t* cell2dof,
-                                const int32_t* adj_ptr, const int32_t* adj, const int32_t* indptr,
-                                const int32_t* indices, int32_t max_row, const void* elem, int64_t elem_stride,
-                                void* values, fa_stream_t stream) {
-    FA_REQUIRE(dtype == FA_F64 || dtype == FA_F32, "fa_gather_matrix: bad dtype %d", dtype);
-    FA_REQUIRE(gdof > 0 && ldof > 0 && max_row > 0, "fa_gather_matrix: bad sizes");
-    const int64_t cs = elem_stride > 0 ? elem_stride : (int64_t)ldof * ldof;
-    FA_REQUIRE(cs >= (int64_t)ldof * ldof, "fa_gather_matrix: element stride %lld < ldof^2", (long long)cs);
-    if (dtype == FA_F64)
-        return dispatch_gather<double>(gdof, ldof, cell2dof, adj_ptr, adj, indptr, indices, max_row, elem, cs, values,
-                                       S(stream));
-    return dispatch_gather<float>(gdof, ldof, cell2dof, adj_ptr, adj, indptr, indices, max_row, elem, cs, values,
-                                  S(stream));
-}
 
 // v[c][i] = sum_j elem[c][i][j] x[c2d[c][j]]: one thread per (cell, row),
 // the row read contiguously, the cell's x entries gathered (shared by the

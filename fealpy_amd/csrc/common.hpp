@@ -100,6 +100,20 @@ __device__ inline unsigned xcd_block() {
 
 inline unsigned xcd_grid(unsigned g) { return (g + 7u) & ~7u; }
 
+// The same within windows of 8 W workgroups (W consecutive ones an XCD), for
+// rows whose work differs along the numbering: a Lagrange space numbers its
+// vertices first, whose rows have several times the incident cells of the
+// others, and one contiguous range an XCD would leave seven waiting for the
+// XCD of the vertices (3.05M P3 rows: 1.46 against 0.96 ms).
+constexpr unsigned XCD_WINDOW = 8;
+
+__device__ inline unsigned xcd_window_block() {
+    const unsigned b = blockIdx.x, in = b % (8 * XCD_WINDOW);
+    return b - in + (in & 7u) * XCD_WINDOW + (in >> 3);
+}
+
+inline unsigned xcd_window_grid(unsigned g) { return (g + 8 * XCD_WINDOW - 1) / (8 * XCD_WINDOW) * (8 * XCD_WINDOW); }
+
 __device__ inline int wave_inclusive_scan(int v) {
     const int lane = threadIdx.x & (WAVE - 1);
 #pragma unroll

@@ -105,6 +105,50 @@ __global__ void __launch_bounds__(256) k_element_vectors(const double* __restric
     }
 }
 
+// out[c][q] = f(x_cq): a thread per point, the block's cells' vertices in LDS
+template <int TD>
+__global__ void __launch_bounds__(256) k_sep_sample(const double* __restrict__ node, const int32_t* __restrict__ cell,
+                                                   int64_t nc, int nq, int cb, const fa_sep_t* __restrict__ se,
+                                                   double* __restrict__ out) {
+    __shared__ double sp[EV_CELLS][TD + 1][TD];
+    __shared__ double sval[SEP_COLS * 256];
+    __shared__ SepPlan plan;
+    sep_plan(se, plan);
+    sep_ones<256>(sval);
+    for (int64_t c0 = (int64_t)blockIdx.x * cb; c0 < nc; c0 += (int64_t)gridDim.x * cb) {
+        const int nb = static_cast<int>(nc - c0 < cb ? nc - c0 : cb);
+        __syncthreads();
+        if (threadIdx.x < nb) {
+            double p[TD + 1][TD];
+            load_cell<TD>(node, cell, c0 + threadIdx.x, p);
+#pragma unroll
+            for (int v = 0; v < TD + 1; ++v)
+#pragma unroll
+                for (int d = 0; d < TD; ++d) sp[threadIdx.x][v][d] = p[v][d];
+        }
+        __syncthreads();
+        for (int t = threadIdx.x; t < nb * nq; t += 256) {
+            const int cl = t / nq, q = t - cl * nq;
+            double f;
+            if (plan.fits) {
+                double x[TD];
+#pragma unroll
+                for (int d = 0; d < TD; ++d) x[d] = 0.0;
+#pragma unroll
+                for (int v = 0; v < TD + 1; ++v) {
+                    const double w = se->bcs[q * (TD + 1) + v];
+#pragma unroll
+                    for (int d = 0; d < TD; ++d) x[d] += w * sp[cl][v][d];
+                }
+                f = sep_value_planned<TD, 256>(se, plan, x, c0 + cl, sval);
+            } else {
+                f = sep_value<TD>(se, q, sp[cl], c0 + cl);
+            }
+            out[c0 * nq + t] = f;
+        }
+    }
+}
+
 // 4 lanes per DOF, lane l adds incidences l, l+4, ...; the lane partials are
 // combined by a fixed tree (deterministic).  A P2-P4 row has 4 to 8
 // incidences on average (an interior DOF of a cell has one), so 16 lanes a
@@ -162,6 +206,22 @@ extern "C" int fa_element_vectors(int dtype, int td, int ldof, int nq, const dou
         else launch_vectors<3, float>(node, cell, nc, ldof, nq, qw, phi, src_kind, src_scale, src, elem, s);
     }
     FA_LAUNCH("k_element_vectors");
+    return FA_OK;
+}
+
+extern "C" int fa_sep_sample(int td, int nq, const double* node, const int32_t* cell, int64_t nc, const void* sep,
+                             double* out, fa_stream_t stream) {
+    FA_REQUIRE(td == 2 || td == 3, "fa_sep_sample: td must be 2 or 3");
+    FA_REQUIRE(nq > 0 && nc >= 0 && sep && out, "fa_sep_sample: bad arguments");
+    if (nc == 0) return FA_OK;
+    const int cb = std::max(1, std::min(EV_CELLS, EV_POINTS / nq));
+    const unsigned grid = grid_for(nc, cb, 256 * 8);
+    const auto* se = static_cast<const fa_sep_t*>(sep);
+    if (td == 2)
+        hipLaunchKernelGGL(k_sep_sample<2>, dim3(grid), dim3(256), 0, S(stream), node, cell, nc, nq, cb, se, out);
+    else
+        hipLaunchKernelGGL(k_sep_sample<3>, dim3(grid), dim3(256), 0, S(stream), node, cell, nc, nq, cb, se, out);
+    FA_LAUNCH("k_sep_sample");
     return FA_OK;
 }
 

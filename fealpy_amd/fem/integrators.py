@@ -231,6 +231,12 @@ def _scalar_elements(space, ops, *, indices=None, selection=_S, dtype=None):
     spec = {'diff': (nat.COEF_NONE, 0.0, None), 'mass': (nat.COEF_NONE, 0.0, None)}
     for op, it in ops:
         spec[op] = coef_spec(it.coef, space, q, selection, allow_sep=True)
+    for op, (kind, scale, table) in spec.items():
+        if kind == nat.COEF_SEP:     # sampled first: the element kernel's registers hold its accumulators
+            vals = torch.empty((nc, qw.shape[0]), dtype=torch.float64, device=space.device)
+            nat.check(L.fa_sep_sample(space.TD, qw.shape[0], nat.ptr(mesh.node), nat.ptr(cell), nc, nat.ptr(table),
+                                      nat.ptr(vals), nat.stream()), "fa_sep_sample")
+            spec[op] = (nat.COEF_CELLQ, scale, vals)
     dtype = torch.float64 if dtype is None else dtype
     elem = torch.empty((nc, ldof, ldof), dtype=dtype, device=space.device)
     (dk, ds, dc), (mk, ms, mc) = spec['diff'], spec['mass']
@@ -360,8 +366,8 @@ def p1_matrix_values(space, ops, pat, dtype):
     for op, it in ops:
         spec[op] = coef_spec(it.coef, space, q, allow_sep=True)
     (dk, ds, dc), (mk, ms, mc) = spec['diff'], spec['mass']
-    values = torch.empty(pat.nnz, dtype=dtype, device=space.device)
     grid = _box_grid(space, pat)
+    values = torch.empty(pat.nnz, dtype=dtype, device=space.device)
     if grid is not None:         # from_box tetrahedra: one pass, cells found from each node's grid position
         nat.check(L.fa_p1_box_matrix(nat.dtype_code(dtype), *grid, nat.ptr(mesh.node_rows16()),
                                      nat.ptr(mesh.box_axes()), qw.shape[0],

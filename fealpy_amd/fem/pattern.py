@@ -29,10 +29,11 @@ def _box_counts(nx, ny, nz):
 
 class Pattern:
     __slots__ = ("cell2dof", "gdof", "ldof", "nc", "_adj_ptr", "_adj", "_max_degree", "indptr", "indices", "nnz",
-                 "max_row", "_maps", "_maps_lock", "_adj_lock")
+                 "max_row", "_maps", "_maps_lock", "_adj_lock", "_pos", "_kept")
 
-    def __init__(self, cell2dof, gdof, box=None):
-        """box: (nx, ny, nz) of a TetrahedronMesh.from_box P1 map, whose CSR
+    def __init__(self, cell2dof, gdof, box=None, kept=False):
+        """kept: the pattern of a space, assembled again and again, which
+        keeps the row positions of its incidences (``row_positions``).  box: (nx, ny, nz) of a TetrahedronMesh.from_box P1 map, whose CSR
         pattern comes from the grid (fa_p1_box_pattern); the incidence lists
         are then built on first use."""
         L = nat.lib()
@@ -44,6 +45,8 @@ class Pattern:
         self._adj_lock = threading.Lock()
         self._maps = None
         self._maps_lock = threading.Lock()
+        self._pos = None
+        self._kept = bool(kept)
         if box is not None:
             nx, ny, nz = box
             self.nnz, self.max_row = _box_counts(nx, ny, nz)
@@ -133,6 +136,34 @@ class Pattern:
         nat.check(st, "fa_incidence_maps")
         return (inc, pos)
 
+    def _positions(self, slot, ldof, longest, build):
+        """Positions of the incidences' columns in their rows, 16 bits each,
+        ldof^2 a cell: built once and completed on the building stream before
+        they are shared.  None for a pattern that is not kept (a region's,
+        summed once: it searches the columns as it sums) or has rows over
+        8192 entries."""
+        if not self._kept or longest > 8192 or self.nnz == 0 or self.nc == 0:
+            return None
+        if getattr(self, slot) is None:
+            with self._maps_lock:
+                if getattr(self, slot) is None:
+                    pos = torch.empty(self.nc * ldof ** 2, dtype=torch.int16, device=self.indptr.device)
+                    build(pos)
+                    torch.cuda.current_stream(pos.device).synchronize()
+                    setattr(self, slot, pos)
+        return getattr(self, slot)
+
+    def row_positions(self):
+        """pos[k*ldof + j] of fa_row_positions (fa_sum_rows)."""
+        if self._pos is not None:
+            return self._pos
+
+        def build(pos):
+            nat.check(nat.lib().fa_row_positions(self.gdof, self.ldof, nat.ptr(self.cell2dof), nat.ptr(self.adj_ptr),
+                                                 nat.ptr(self.adj), nat.ptr(self.indptr), nat.ptr(self.indices),
+                                                 self.max_row, nat.ptr(pos), nat.stream()), "fa_row_positions")
+        return self._positions('_pos', self.ldof, self.max_row, build)
+
     def gather_matrix(self, elem, values=None):
         """CSR values from element matrices (NC, ldof, ldof) in ascending-cell order."""
         L = nat.lib()
@@ -142,6 +173,12 @@ class Pattern:
             elem = elem.contiguous()                      # cells may be padded apart; rows must be dense
         if values is None:
             values = torch.empty(self.nnz, dtype=elem.dtype, device=elem.device)
+        pos = self.row_positions()
+        if pos is not None:
+            nat.check(L.fa_sum_rows(nat.dtype_code(elem.dtype), self.gdof, self.ldof, nat.ptr(self.adj_ptr),
+                                    nat.ptr(self.adj), nat.ptr(self.indptr), nat.ptr(pos), self.max_row, nat.ptr(elem),
+                                    elem.stride(0), nat.ptr(values), nat.stream()), "fa_sum_rows")
+            return values
         nat.check(L.fa_gather_matrix(nat.dtype_code(elem.dtype), self.gdof, self.ldof, nat.ptr(self.cell2dof),
                                      nat.ptr(self.adj_ptr), nat.ptr(self.adj), nat.ptr(self.indptr),
                                      nat.ptr(self.indices), max(self.max_row, 1), nat.ptr(elem), elem.stride(0),
@@ -186,7 +223,8 @@ def pattern_of(space, cell2dof=None):
         if getattr(space, "_pattern", None) is None:
             with _LOCK:
                 if getattr(space, "_pattern", None) is None:
-                    pat = Pattern(space.cell_to_dof(), space.number_of_global_dofs(), box=_box_grid_of(space))
+                    pat = Pattern(space.cell_to_dof(), space.number_of_global_dofs(), box=_box_grid_of(space),
+                                  kept=True)
                     torch.cuda.current_stream(pat.indptr.device).synchronize()
                     space._pattern = pat
         return space._pattern

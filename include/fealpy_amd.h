@@ -166,6 +166,16 @@ int fa_gather_matrix(int dtype, int64_t gdof, int32_t ldof, const int32_t* cell2
                      const int32_t* adj_ptr, const int32_t* adj,
                      const int32_t* indptr, const int32_t* indices, int32_t max_row,
                      const void* elem, int64_t elem_stride, void* values, fa_stream_t stream);
+/* The same sum for a pattern that is assembled again and again: positions
+ * (fa_row_positions, once per pattern) of each incidence's columns in its
+ * CSR row, pos[k*ldof + j] for incidence k (in adj order).  Same order of
+ * every sum, in FP64. */
+int fa_row_positions(int64_t gdof, int32_t ldof, const int32_t* cell2dof, const int32_t* adj_ptr,
+                     const int32_t* adj, const int32_t* indptr, const int32_t* indices, int32_t max_row,
+                     uint16_t* pos, fa_stream_t stream);
+int fa_sum_rows(int dtype, int64_t gdof, int32_t ldof, const int32_t* adj_ptr, const int32_t* adj,
+                const int32_t* indptr, const uint16_t* pos, int32_t max_row, const void* elem, int64_t elem_stride,
+                void* values, fa_stream_t stream);
 /* Dense global vector from element vectors: LinearForm.assembly(format='dense')
  * (fealpy/fem/linear_form.py:66-86 -> COOTensor.to_dense, coo_tensor.py:116-130). */
 int fa_gather_vector(int dtype, int64_t gdof, int32_t ldof,
@@ -270,6 +280,14 @@ int fa_p1_box_matrix(int dtype, int nx, int ny, int nz, const double* node_wide,
  * LagrangeFESpace.boundary_interpolate does with gd
  * (fealpy/functionspace/lagrange_fe_space.py:109-140), in one launch. */
 int fa_sep_points(const void* sep, int64_t n, int gd, const double* points, double* out, fa_stream_t stream);
+
+/* f at the quadrature points of every cell: out[c*nq + q] = f(x_cq) for an
+ * fa_sep_t in device memory (its `bcs` is the (nq, td+1) table of the rule),
+ * the (NC, NQ) array of a FA_COEF_CELLQ coefficient.  Replaces the
+ * reference's evaluation of a @cartesian coefficient at
+ * mesh.bc_to_point(bcs) (fealpy/utils/utils.py:21-53). */
+int fa_sep_sample(int td, int nq, const double* node, const int32_t* cell, int64_t nc, const void* sep, double* out,
+                  fa_stream_t stream);
 
 /* Grid lines of a from_box node array: axes[0 .. nx] = x of nodes (i, 0, 0),
  * then y of (0, j, 0), then z of (0, 0, k) (nx + ny + nz + 3 doubles), and
