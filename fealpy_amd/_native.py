@@ -43,6 +43,14 @@ _SIGNATURES = {
     "fa_gather_matrix": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _p, _i32, _p, _i64, _p, _p]),
     "fa_row_positions": (ctypes.c_int, [_i64, _i32, _p, _p, _p, _p, _p, _i32, _p, _p]),
     "fa_sum_rows": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _i32, _p, _i64, _p, _p]),
+    "fa_p1_records_bytes": (_sz, [ctypes.c_int, _i64]),
+    "fa_assemble_p1_rows": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _i64, _i64, _p, _p, _p, ctypes.c_int, _f64, _p,
+                                           ctypes.c_int, _f64, _p, _p, _p, _p, _p, _i32, _p, _sz, _p, _p]),
+    "fa_vector_positions": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _p, _i32, _p, _p]),
+    "fa_elasticity_records_bytes": (_sz, [ctypes.c_int, _i64]),
+    "fa_assemble_elasticity_rows": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _i64, _i64, _i32, _p, _p,
+                                                   _p, _f64, _f64, _f64, _f64, _p, _p, _p, _i64, _p, _i32, _p, _sz,
+                                                   _p, _p]),
     "fa_gather_vector": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _p, _p, _p]),
     "fa_element_apply": (ctypes.c_int, [ctypes.c_int, _i64, _i32, _p, _p, _i64, _p, _p, _p]),
     "fa_element_elasticity": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p, _i64, _p,

@@ -104,7 +104,8 @@ inline unsigned xcd_grid(unsigned g) { return (g + 7u) & ~7u; }
 // rows whose work differs along the numbering: a Lagrange space numbers its
 // vertices first, whose rows have several times the incident cells of the
 // others, and one contiguous range an XCD would leave seven waiting for the
-// XCD of the vertices (3.05M P3 rows: 1.46 against 0.96 ms).
+// XCD of the vertices (P2 elasticity at 40^3: 1.8 against
+// 0.6 ms, 3.05M P3 rows 1.46 against 0.96 ms).
 constexpr unsigned XCD_WINDOW = 8;
 
 __device__ inline unsigned xcd_window_block() {

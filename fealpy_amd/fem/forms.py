@@ -9,6 +9,8 @@ import torch
 
 from .. import _native as nat
 from ..sparse.tensors import COOTensor, CSRTensor
+from . import rows
+from .elasticity import LinearElasticityIntegrator
 from .integrators import GroupIntegrator, Integrator, _axpby_sum, _call_assembly, coef_spec, p1_fusable_ops, \
     p1_matrix_values, p1_source_fusable, p1_vector_values
 from .pattern import pattern_of
@@ -113,6 +115,10 @@ class BilinearForm(Form):
         if fused is not None:
             self._M = fused if format == 'csr' else fused.tocoo()
             return self._M
+        fused = self._elasticity_rows(space, dtype) if hasattr(space, 'scalar_space') else None
+        if fused is not None:
+            self._M = fused if format == 'csr' else fused.tocoo()
+            return self._M
         full_map = space.cell_to_dof()
         total = None
         values = None
@@ -150,6 +156,23 @@ class BilinearForm(Form):
         for ops in groups:
             v = p1_matrix_values(space, ops, pat, dtype)
             values = v if values is None else _axpby_sum(values, v)
+        return CSRTensor(pat.indptr, pat.indices, values, self.sparse_shape)
+
+    def _elasticity_rows(self, space, dtype):
+        """One elasticity integrator over all cells of a vector space: rows
+        summed from a record per cell (rows.py), no element matrices."""
+        ints = list(self.integrators.values())
+        dtype = torch.float64 if dtype is None else dtype
+        if len(ints) != 1 or dtype not in (torch.float64, torch.float32):
+            return None
+        it = ints[0]
+        if type(it) is not LinearElasticityIntegrator or it.get_region() is not None or space.dof_ndim != 1 \
+                or space.dof_numel != space.GD or space.GD != space.TD:
+            return None
+        values = rows.elasticity_values(space, it, dtype)
+        if values is None:
+            return None
+        pat = pattern_of(space)
         return CSRTensor(pat.indptr, pat.indices, values, self.sparse_shape)
 
     def __matmul__(self, u):

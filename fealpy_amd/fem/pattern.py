@@ -29,7 +29,7 @@ def _box_counts(nx, ny, nz):
 
 class Pattern:
     __slots__ = ("cell2dof", "gdof", "ldof", "nc", "_adj_ptr", "_adj", "_max_degree", "indptr", "indices", "nnz",
-                 "max_row", "_maps", "_maps_lock", "_adj_lock", "_pos", "_kept")
+                 "max_row", "_maps", "_maps_lock", "_adj_lock", "_pos", "_vpos", "_kept")
 
     def __init__(self, cell2dof, gdof, box=None, kept=False):
         """kept: the pattern of a space, assembled again and again, which
@@ -45,7 +45,7 @@ class Pattern:
         self._adj_lock = threading.Lock()
         self._maps = None
         self._maps_lock = threading.Lock()
-        self._pos = None
+        self._pos = self._vpos = None
         self._kept = bool(kept)
         if box is not None:
             nx, ny, nz = box
@@ -154,7 +154,7 @@ class Pattern:
         return getattr(self, slot)
 
     def row_positions(self):
-        """pos[k*ldof + j] of fa_row_positions (fa_sum_rows)."""
+        """pos[k*ldof + j] of fa_row_positions (fa_sum_rows, fa_assemble_p1_rows)."""
         if self._pos is not None:
             return self._pos
 
@@ -163,6 +163,19 @@ class Pattern:
                                                  nat.ptr(self.adj), nat.ptr(self.indptr), nat.ptr(self.indices),
                                                  self.max_row, nat.ptr(pos), nat.stream()), "fa_row_positions")
         return self._positions('_pos', self.ldof, self.max_row, build)
+
+    def vector_positions(self, td, dof_priority):
+        """The positions of a vector space's scalar incidences (fa_vector_positions)."""
+        if self._vpos is not None:
+            return self._vpos
+        ldof = self.ldof // td
+
+        def build(pos):
+            nat.check(nat.lib().fa_vector_positions(td, int(dof_priority), self.gdof // td, ldof,
+                                                    nat.ptr(self.cell2dof), nat.ptr(self.adj_ptr), nat.ptr(self.adj),
+                                                    nat.ptr(self.indptr), nat.ptr(self.indices), self.max_row,
+                                                    nat.ptr(pos), nat.stream()), "fa_vector_positions")
+        return self._positions('_vpos', ldof, self.max_row // td, build)
 
     def gather_matrix(self, elem, values=None):
         """CSR values from element matrices (NC, ldof, ldof) in ascending-cell order."""

@@ -176,6 +176,39 @@ int fa_row_positions(int64_t gdof, int32_t ldof, const int32_t* cell2dof, const 
 int fa_sum_rows(int dtype, int64_t gdof, int32_t ldof, const int32_t* adj_ptr, const int32_t* adj,
                 const int32_t* indptr, const uint16_t* pos, int32_t max_row, const void* elem, int64_t elem_stride,
                 void* values, fa_stream_t stream);
+/* CSR values of P1 scalar diffusion + mass with coefficients constant on each
+ * cell: a record per cell (the entries i <= j of its matrix; `records`,
+ * fa_p1_records_bytes), then each row summed over its incident cells in
+ * ascending order.  Replaces the same loop as fa_element_matrices +
+ * fa_gather_matrix (scalar_diffusion_integrator.py:25-63,
+ * scalar_mass_integrator.py:23-54, coo_tensor.py:184-213).
+ * table (NS+1, td+1, td+1) FP64: for the NS = td (td+1)/2 pairs (a, b), a <= b,
+ * in row order, sum_q w_q (R'_ia R'_jb + [a != b] R'_ib R'_ja) with
+ * R' = R[:, :, 1:] - R[:, :, :1]; last, sum_q w_q phi_i phi_j.
+ * node_wide: 16-byte rows (2 doubles in 2D, 4 in 3D); cell: (NC, td+1) vertices;
+ * pos as fa_row_positions. */
+size_t fa_p1_records_bytes(int td, int64_t nc);
+int fa_assemble_p1_rows(int dtype, int td, int64_t gdof, int64_t nc, const double* node_wide, const int32_t* cell,
+                        const double* table, int diff_kind, double diff_scale, const double* diff_coef, int mass_kind,
+                        double mass_scale, const double* mass_coef, const int32_t* adj_ptr, const int32_t* adj,
+                        const int32_t* indptr, const uint16_t* pos, int32_t max_row, void* records,
+                        size_t records_bytes, void* values, fa_stream_t stream);
+/* CSR values of isotropic linear elasticity, without element matrices, on a vector space (td components)
+ * over ndof scalar DOFs of ldof a cell, in either DOF layout: replaces
+ * fa_element_elasticity + fa_gather_matrix
+ * (linear_elasticity_integrator.py:90-165).  adj_ptr, adj, indptr: the vector
+ * space's own lists; pos: fa_vector_positions (places of a scalar incidence's
+ * scalar columns); max_row: its longest row.  table (td, td, ldof, ldof):
+ * sum_q w_q R'_ia R'_jb.  cA..cD as fa_element_elasticity. */
+int fa_vector_positions(int td, int dof_priority, int64_t ndof, int32_t ldof, const int32_t* cell2dof,
+                        const int32_t* adj_ptr, const int32_t* adj, const int32_t* indptr, const int32_t* indices,
+                        int32_t max_row, uint16_t* pos, fa_stream_t stream);
+size_t fa_elasticity_records_bytes(int td, int64_t nc);
+int fa_assemble_elasticity_rows(int dtype, int td, int dof_priority, int64_t ndof, int64_t nc, int32_t ldof,
+                                const double* node_wide, const int32_t* cell, const double* table, double cA,
+                                double cB, double cC, double cD, const int32_t* adj_ptr, const int32_t* adj,
+                                const int32_t* indptr, int64_t nnz, const uint16_t* pos, int32_t max_row,
+                                void* records, size_t records_bytes, void* values, fa_stream_t stream);
 /* Dense global vector from element vectors: LinearForm.assembly(format='dense')
  * (fealpy/fem/linear_form.py:66-86 -> COOTensor.to_dense, coo_tensor.py:116-130). */
 int fa_gather_vector(int dtype, int64_t gdof, int32_t ldof,

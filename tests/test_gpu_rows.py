@@ -1,0 +1,87 @@
+"""Rows summed from a record per cell (fa_assemble_p1_rows,
+fa_assemble_elasticity_rows) against the element matrices of the same forms,
+summed in FP64 on the CPU: meshes with shuffled numbering, a vertex of high
+degree, the smallest meshes, both value types and DOF layouts.  An entry adds at
+most `deg` cells' values, each a sum of at most 9 products on either side:
+9 deg units in the last place of the largest entry."""
+import numpy as np
+import pytest
+import torch
+
+import fealpy_amd as fa
+from fealpy_amd.fem import integrators, rows
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+
+
+def _shuffled(mesh, seed):
+    g = np.random.default_rng(seed)
+    node, cell = mesh.node.cpu().numpy(), mesh.cell.cpu().numpy()
+    perm = g.permutation(len(node))
+    new = np.empty_like(perm)
+    new[perm] = np.arange(len(node))
+    return type(mesh)(torch.as_tensor(node[perm], device=DEV), torch.as_tensor(new[cell][g.permutation(len(cell))],
+                                                                              dtype=torch.int32, device=DEV))
+
+
+def _fan(n):
+    """n triangles around one vertex: a row of n + 1 entries and n incidences."""
+    t = 2 * np.pi * np.arange(n) / n
+    node = np.concatenate([[[0.0, 0.0]], np.stack([np.cos(t), np.sin(t)], 1)])
+    cell = np.stack([np.zeros(n, int), 1 + np.arange(n), 1 + (np.arange(n) + 1) % n], 1)
+    return fa.TriangleMesh(torch.as_tensor(node, device=DEV), torch.as_tensor(cell, dtype=torch.int32, device=DEV))
+
+
+MESHES = {"tri1": lambda: fa.TriangleMesh.from_box(nx=1, ny=1, device=DEV),
+          "tri": lambda: _shuffled(fa.TriangleMesh.from_box(nx=9, ny=7, device=DEV), 1),
+          "fan": lambda: _fan(300),
+          "tet1": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=1, ny=1, nz=1, device=DEV), 2),
+          "tet": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=4, ny=3, nz=5, device=DEV), 3)}
+
+
+def _dense(space, elem):
+    n = space.number_of_global_dofs()
+    c2d = space.cell_to_dof().cpu().long()
+    out = torch.zeros(n * n, dtype=torch.float64)
+    out.index_add_(0, (c2d[:, :, None] * n + c2d[:, None, :]).reshape(-1), elem.cpu().reshape(-1))
+    return out.reshape(n, n), int(torch.bincount(c2d.reshape(-1)).max())
+
+
+def _check(A, space, elem, dtype):
+    ref, deg = _dense(space, elem)
+    eps = 9 * deg * 2.2e-16 + (6e-8 if dtype == torch.float32 else 0.0)
+    assert A.values.dtype == dtype
+    assert float((A.to_dense().cpu().double() - ref).abs().max()) <= eps * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("name", sorted(MESHES))
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("ops", ["diff", "mass", "both"])
+def test_p1_rows(name, dtype, ops, monkeypatch):
+    monkeypatch.setattr(integrators, "RECORDS_MIN_CELLS", 0)
+    mesh = MESHES[name]()
+    space = fa.LagrangeFESpace(mesh, 1)
+    k = torch.as_tensor(np.exp(np.random.default_rng(4).standard_normal(mesh.number_of_cells())), device=DEV)
+    ints = [fa.ScalarDiffusionIntegrator(k, q=3)] if ops != "mass" else []
+    ints += [fa.ScalarMassIntegrator(0.5 if ops == "both" else k, q=3)] if ops != "diff" else []
+    group = fa.GroupIntegrator(*ints)
+    A = fa.BilinearForm(space).add_integrator(group).assembly(dtype=dtype)
+    _check(A, space, group.assembly(space), dtype)
+
+
+@pytest.mark.parametrize("name,p", [("tri1", 1), ("tri", 1), ("tri", 2), ("fan", 2), ("tri", 3), ("tri", 4), ("tet1", 1),
+                                    ("tet", 1), ("tet1", 2), ("tet", 2), ("tet", 3)])
+@pytest.mark.parametrize("prio", [False, True])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_elasticity_rows(name, p, prio, dtype, monkeypatch):
+    monkeypatch.setattr(rows, "ELASTICITY_MIN_DOFS", 0)
+    mesh = MESHES[name]()
+    gd = mesh.geo_dimension()
+    space = fa.TensorFunctionSpace(fa.LagrangeFESpace(mesh, p), (gd, -1) if prio else (-1, gd))
+    mat = fa.LinearElasticMaterial("m", lame_lambda=1.3, shear_modulus=0.7,
+                                   **({} if gd == 3 else {"hypo": "plane_strain"}))
+    it = fa.LinearElasticityIntegrator(mat, q=p + 2)
+    assert rows.elasticity_values(space, it, dtype) is not None
+    A = fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype)
+    _check(A, space, it.assembly(space), dtype)
