@@ -124,6 +124,9 @@ _SIGNATURES = {
     "fa_p1_box_pattern": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p, _i64, _p, _sz, _p]),
     "fa_p1_box_vector": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, ctypes.c_int, _p,
                                         _p, ctypes.c_int, _f64, _p, _p, _p, _sz, _p]),
+    "fa_p1_box_vector_tensor_work_bytes": (_sz, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int]),
+    "fa_p1_box_vector_tensor": (ctypes.c_int, [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, _p, _p,
+                                               ctypes.c_int, _p, _p, _f64, _p, _p, _p, _sz, _p]),
     "fa_p1_incidence_vectors": (ctypes.c_int, [ctypes.c_int, _i64, ctypes.c_int, _p, _p, _p, _p, ctypes.c_int, _f64,
                                                _p, _p, _p, _p]),
     "fa_sum_incidence_values": (ctypes.c_int, [ctypes.c_int, _i64, _p, _p, _p, _p]),

@@ -1,5 +1,6 @@
 // Kernels "a" and "c": element matrices / vectors on simplices and the
 // fixed-order (ascending cell) gather of element contributions into CSR rows.
+#include "box.hpp"
 #include "cell.hpp"
 #include "common.hpp"
 #include "reduce.hpp"
@@ -1099,59 +1100,6 @@ extern "C" int fa_sum_incidence_values(int dtype, int64_t gdof, const int32_t* a
 // CSR row (some cube holds the pair as a Kuhn edge), and ascending column
 // order is lexicographic offset order, so the entry's position in the row is
 // the number of present neighbours before it.
-// offsets of corner k as bit masks over k (corners 1, 2, 5, 6 have x + 1;
-// 2, 3, 6, 7 have y + 1; 4-7 have z + 1): branch-free for a runtime k
-constexpr int box_cdx(int k) { return (0x66 >> k) & 1; }
-constexpr int box_cdy(int k) { return (0xCC >> k) & 1; }
-constexpr int box_cdz(int k) { return (k >> 2) & 1; }
-constexpr int box_corner_of(int a, int b, int c) {
-    return c == 0 ? (a == 0 ? (b == 0 ? 0 : 3) : (b == 0 ? 1 : 2)) : (a == 0 ? (b == 0 ? 4 : 7) : (b == 0 ? 5 : 6));
-}
-constexpr int box_kuhn(int t, int v) {
-    constexpr int K[6][4] = {{0, 1, 2, 6}, {0, 5, 1, 6}, {0, 4, 5, 6}, {0, 7, 4, 6}, {0, 3, 7, 6}, {0, 2, 3, 6}};
-    return K[t][v];
-}
-// local index of corner k in tetrahedron t, or -1
-constexpr int box_local(int t, int k) {
-    return box_kuhn(t, 0) == k ? 0 : box_kuhn(t, 1) == k ? 1 : box_kuhn(t, 2) == k ? 2 : box_kuhn(t, 3) == k ? 3 : -1;
-}
-// accumulator slot of offset (dx, dy, dz): rank among the 15 offsets in
-// lexicographic order, -1 for an offset that is no Kuhn edge
-constexpr int box_slot(int dx, int dy, int dz) {
-    constexpr int S[27] = {0, 1, -1, 2, 3, -1, -1, -1, -1, 4, 5, -1, 6, 7, 8, -1, 9, 10,
-                           -1, -1, -1, -1, 11, 12, -1, 13, 14};
-    return S[(dx + 1) * 9 + (dy + 1) * 3 + (dz + 1)];
-}
-constexpr int BOX_SLOTS = 15;
-
-// Kuhn tetrahedra as paths: the corners of tetrahedron t, ordered by their
-// number of +1 offsets, run from corner 0 to corner 6 one axis at a time.
-// box_pos: path position of local vertex v; box_axis: the axis of path step
-// p (1..3); box_sign: orientation of the local vertex order (the sign of
-// det(o1 - o0, o2 - o0, o3 - o0) on the unit cube)
-constexpr int box_pos(int t, int v) {
-    return box_cdx(box_kuhn(t, v)) + box_cdy(box_kuhn(t, v)) + box_cdz(box_kuhn(t, v));
-}
-constexpr int box_corner_at(int t, int p) {
-    return box_pos(t, 0) == p ? box_kuhn(t, 0)
-           : box_pos(t, 1) == p ? box_kuhn(t, 1)
-           : box_pos(t, 2) == p ? box_kuhn(t, 2)
-                                : box_kuhn(t, 3);
-}
-constexpr int box_axis(int t, int p) {
-    return box_cdx(box_corner_at(t, p)) != box_cdx(box_corner_at(t, p - 1))   ? 0
-           : box_cdy(box_corner_at(t, p)) != box_cdy(box_corner_at(t, p - 1)) ? 1
-                                                                               : 2;
-}
-constexpr int box_off(int t, int v, int d) {
-    return (d == 0 ? box_cdx(box_kuhn(t, v)) : d == 1 ? box_cdy(box_kuhn(t, v)) : box_cdz(box_kuhn(t, v))) -
-           (d == 0 ? box_cdx(box_kuhn(t, 0)) : d == 1 ? box_cdy(box_kuhn(t, 0)) : box_cdz(box_kuhn(t, 0)));
-}
-constexpr int box_sign(int t) {
-    return box_off(t, 1, 0) * (box_off(t, 2, 1) * box_off(t, 3, 2) - box_off(t, 2, 2) * box_off(t, 3, 1)) -
-           box_off(t, 1, 1) * (box_off(t, 2, 0) * box_off(t, 3, 2) - box_off(t, 2, 2) * box_off(t, 3, 0)) +
-           box_off(t, 1, 2) * (box_off(t, 2, 0) * box_off(t, 3, 1) - box_off(t, 2, 1) * box_off(t, 3, 0));
-}
 
 // the contributions of the tetrahedra of cube (ix - A, iy - B, iz - C) that
 // hold the node, in ascending cell order
@@ -1381,6 +1329,17 @@ __global__ void __launch_bounds__(256) k_box_sep_table(int nx, int ny, int nz, c
         }
         tab[idx] = sep_factor(e->kind[k], e->a[k], e->b[k], x);
     }
+}
+
+int fa::launch_box_sep_table(int nx, int ny, int nz, const double* node_wide, const void* sep, int nq, double* axes,
+                             double* tab, hipStream_t s) {
+    const int nmax = std::max(nx, std::max(ny, nz));
+    // the table's size follows the struct's factor count, read on the device
+    const int64_t most = static_cast<int64_t>(nx) + ny + nz + 3 + static_cast<int64_t>(FA_SEP_MAX_FACTORS) * nmax * 6 * nq;
+    hipLaunchKernelGGL(k_box_sep_table, dim3(grid_for(most, 256, 1 << 14)), dim3(256), 0, s, nx, ny, nz, node_wide,
+                       static_cast<const fa_sep_t*>(sep), nq, nmax, axes, tab);
+    FA_LAUNCH("k_box_sep_table");
+    return FA_OK;
 }
 
 // sep_value at the NQ points of each of the 6 tetrahedra of cube (cx, cy,
@@ -2248,12 +2207,9 @@ extern "C" int fa_p1_box_vector(int dtype, int nx, int ny, int nz, const double*
     hipStream_t s = S(stream);
     const bool sep = src_kind == FA_COEF_SEP;
     timer_begin(FA_TIMER_P1_VECTORS, s);
-    if (sep) {  // the table's size follows the struct's factor count, read on the device
-        const int64_t most = static_cast<int64_t>(nx) + ny + nz + 3 +
-                             static_cast<int64_t>(FA_SEP_MAX_FACTORS) * nmax * 6 * nq;
-        hipLaunchKernelGGL(k_box_sep_table, dim3(grid_for(most, 256, 1 << 14)), dim3(256), 0, s, nx, ny, nz,
-                           node_wide, reinterpret_cast<const fa_sep_t*>(src), nq, nmax, axes, tab);
-        FA_LAUNCH("k_box_sep_table");
+    if (sep) {
+        const int st = launch_box_sep_table(nx, ny, nz, node_wide, src, nq, axes, tab, s);
+        if (st != FA_OK) return st;
     }
     const unsigned g1 = grid_for(nc / 6, 256, 1 << 20);
     if (sep)

@@ -421,6 +421,13 @@ def p1_vector_values(space, it, pat, dtype):
         kind, scale, src = nat.COEF_CONST, 1.0, None
     out = torch.empty(pat.gdof, dtype=dtype, device=space.device)
     grid = _box_grid(space, pat)
+    axes = mesh.box_axes() if grid is not None and kind == nat.COEF_SEP else None
+    if axes is not None:         # a separable source on a tensor grid: one pass
+        work = nat.workspace(L.fa_p1_box_vector_tensor_work_bytes(*grid, qw.shape[0]), space.device)
+        nat.check(L.fa_p1_box_vector_tensor(nat.dtype_code(dtype), *grid, nat.ptr(mesh.node_rows16()), nat.ptr(axes),
+                                            qw.shape[0], nat.ptr(qw), nat.ptr(phi), scale, nat.ptr(src), nat.ptr(out),
+                                            nat.ptr(work), work.numel(), nat.stream()), "fa_p1_box_vector_tensor")
+        return out
     if grid is not None:         # from_box tetrahedra: cell-order element vectors, then a gather per node by grid position
         work = nat.workspace(L.fa_p1_box_vector_work_bytes(*grid, qw.shape[0]), space.device)
         nat.check(L.fa_p1_box_vector(nat.dtype_code(dtype), *grid, nat.ptr(mesh.node_rows16()), qw.shape[0],

@@ -306,6 +306,15 @@ int fa_p1_box_matrix(int dtype, int nx, int ny, int nz, const double* node_wide,
                      int mass_kind, double mass_scale, const double* mass_coef, const int32_t* indptr, int64_t nnz,
                      void* values, fa_stream_t stream);
 
+/* fa_p1_box_vector for a separable source (scale * sep, an fa_sep_t in device
+ * memory) on a grid whose nodes lie on the grid lines `axes` (fa_box_axes with
+ * *on_grid_host = 1), in one pass and without the element-vector buffer: the
+ * same sums in the same order, equal to a few units in the last place. */
+size_t fa_p1_box_vector_tensor_work_bytes(int nx, int ny, int nz, int nq);
+int fa_p1_box_vector_tensor(int dtype, int nx, int ny, int nz, const double* node_wide, const double* axes, int nq,
+                            const double* qw, const double* phi, double scale, const void* sep, void* out, void* work,
+                            size_t work_bytes, fa_stream_t stream);
+
 /* f at n cartesian points (points[n*gd], row-major, FP64) for a field-free
  * fa_sep_t in device memory (its field pointers and bcs are not read):
  * out[i] = sum_t coef[t] prod_k g_k(points[i*gd + dim[k]]).  Replaces the

@@ -1,0 +1,43 @@
+"""One-pass load vector of a separable source on a tensor grid
+(fa_p1_box_vector_tensor) against the kernels of any other mesh: grids around
+the block's tile (7 x 31 nodes, chunks of planes), one term and several, the
+one-, four- and eleven-point rules, a field, FP32 results.  Both sides add the
+same products (up to 24 cells of NQ points, four factors each) in the same cell
+order, so they differ by (NQ + 24 + 4) units in the last place at most."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+import fealpy_amd as fa
+from fealpy_amd import expr
+from fealpy_amd.fem import integrators
+
+pytestmark = pytest.mark.gpu
+DEV = torch.device("cuda")
+PI = math.pi
+
+
+def _source(name, nc):
+    x, y, z = expr.x, expr.y, expr.z
+    one = expr.sin(PI * x + 0.3) * expr.cos(PI * y) * expr.exp(0.5 * z)
+    k = torch.as_tensor(np.exp(np.random.default_rng(nc).standard_normal(nc)), device=DEV)
+    return {"one": 2.0 * one, "field": 3.0 * expr.cell(k) * one * expr.sin(2.0 * x), "plane": expr.sin(PI * y + 0.1),
+            "terms": 2.0 * expr.cell(k) * one + expr.sin(2.0 * z) * expr.x + 0.5}[name]
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 6, 30), (5, 7, 31), (3, 8, 32), (9, 13, 3), (17, 2, 62)])
+@pytest.mark.parametrize("q", [1, 2, 4])
+@pytest.mark.parametrize("name", ["one", "field", "plane", "terms"])
+def test_tensor_grid_load_vector(dims, q, name, monkeypatch):
+    mesh = fa.TetrahedronMesh.from_box([0, 1, 0, 2, -1, 1], nx=dims[0], ny=dims[1], nz=dims[2], device=DEV)
+    space = fa.LagrangeFESpace(mesh, 1)
+    form = fa.LinearForm(space).add_integrator(fa.ScalarSourceIntegrator(_source(name, mesh.number_of_cells()), q=q))
+    got = form.assembly()
+    assert torch.equal(form.assembly(dtype=torch.float32), got.to(torch.float32))
+    assert torch.equal(form.assembly(), got)
+    monkeypatch.setattr(integrators, "BOX_ASSEMBLY", False)
+    ref = form.assembly()
+    nq = mesh.quadrature_formula(q).get_quadrature_points_and_weights()[1].shape[0]
+    assert float((got - ref).abs().max()) <= (nq + 28) * 2.2e-16 * float(ref.abs().max())
