@@ -8,32 +8,69 @@
 namespace fa {
 
 // ---- SpMV -------------------------------------------------------------------
+// A block takes 256 / G consecutive rows, whose entries are one contiguous
+// range: it reads that range whole lines at a time whatever the rows' lengths,
+// four entries a thread in flight, leaves the products in LDS, and G lanes a
+// row add the row's.  What bounds it is HBM: 12 (8 in FP32) bytes an entry.
+// The form with G lanes reading each row themselves lost them in the rows'
+// remainders and waited for one entry at a time: a P2 tetrahedral matrix
+// (885k rows of 18 to 65 entries, FP64) 141 -> 73 us, 4.4 TB/s.
+constexpr int STREAM = 2048;  // products held at once
+
 template <class T, int G>
 __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t* __restrict__ indptr,
                                              const int32_t* __restrict__ indices, const T* __restrict__ vals,
                                              const T* __restrict__ x, T* __restrict__ y) {
+    constexpr int RB = 256 / G;
+    __shared__ T prod[STREAM];
     const int lane = threadIdx.x % G;
-    for (int64_t r = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / G; r < n;
-         r += (int64_t)gridDim.x * blockDim.x / G) {
-        const int32_t k1 = indptr[r + 1];
+    for (int64_t r0 = (int64_t)xcd_window_block() * RB; r0 < n; r0 += (int64_t)gridDim.x * RB) {
+        const int64_t end = min(r0 + RB, n), r = min(r0 + threadIdx.x / G, end);
+        const int32_t e0 = indptr[r0], e1 = indptr[end];
+        const int32_t k0 = indptr[r], k1 = indptr[min(r + 1, end)];
         T s = T(0);
-        for (int32_t k = indptr[r] + lane; k < k1; k += G) s += vals[k] * x[indices[k]];
+        for (int32_t e = e0; e < e1; e += STREAM) {
+            const int m = min(STREAM, e1 - e);
+            for (int b = 0; b < m; b += 1024) {
+                int32_t c[4];
+                T v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int32_t k = e + min(b + u * 256 + (int)threadIdx.x, m - 1);
+                    c[u] = indices[k];
+                    v[u] = vals[k];
+                }
+                T w[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) w[u] = x[c[u]];
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (b + u * 256 + (int)threadIdx.x < m) prod[b + u * 256 + threadIdx.x] = v[u] * w[u];
+            }
+            __syncthreads();
+            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s += prod[k - e];
+            __syncthreads();
+        }
         s = group_sum<G>(s);
-        if (lane == 0) y[r] = s;
+        if (lane == 0 && r < end) y[r] = s;
     }
 }
 
 template <class T>
 static int spmv_launch(int64_t n, const int32_t* indptr, const int32_t* indices, const T* vals, const T* x, T* y,
                        int G, hipStream_t s) {
-    const unsigned grid = grid_for(n * G, 256, 1 << 20);
+    const unsigned grid = xcd_window_grid(grid_for(n * G, 256, 1 << 20));
+    auto k = k_spmv<T, 64>;
     switch (G) {
-        case 4: hipLaunchKernelGGL((k_spmv<T, 4>), dim3(grid), dim3(256), 0, s, n, indptr, indices, vals, x, y); break;
-        case 8: hipLaunchKernelGGL((k_spmv<T, 8>), dim3(grid), dim3(256), 0, s, n, indptr, indices, vals, x, y); break;
-        case 16: hipLaunchKernelGGL((k_spmv<T, 16>), dim3(grid), dim3(256), 0, s, n, indptr, indices, vals, x, y); break;
-        case 32: hipLaunchKernelGGL((k_spmv<T, 32>), dim3(grid), dim3(256), 0, s, n, indptr, indices, vals, x, y); break;
-        default: hipLaunchKernelGGL((k_spmv<T, 64>), dim3(grid), dim3(256), 0, s, n, indptr, indices, vals, x, y); break;
+        case 1: k = k_spmv<T, 1>; break;
+        case 2: k = k_spmv<T, 2>; break;
+        case 4: k = k_spmv<T, 4>; break;
+        case 8: k = k_spmv<T, 8>; break;
+        case 16: k = k_spmv<T, 16>; break;
+        case 32: k = k_spmv<T, 32>; break;
+        default: break;
     }
+    hipLaunchKernelGGL(k, dim3(grid), dim3(256), 0, s, n, indptr, indices, vals, x, y);
     FA_LAUNCH("k_spmv");
     return FA_OK;
 }
@@ -69,13 +106,13 @@ __global__ void __launch_bounds__(256) k_spmm(int64_t n, int64_t nv, const int32
     }
 }
 
+// lanes per row: so many that a block's 256 / G rows hold one to two
+// thousand entries on average
 static int lanes_for(int64_t n, int64_t nnz) {
     const double avg = n > 0 ? double(nnz) / double(n) : 1.0;
-    if (avg <= 6) return 4;
-    if (avg <= 12) return 8;
-    if (avg <= 24) return 16;
-    if (avg <= 48) return 32;
-    return 64;
+    int g = 1;
+    while (g < 64 && 8.0 * g < avg) g <<= 1;
+    return g;
 }
 
 // ---- Dirichlet BC (G lanes per row) ------------------------------------------------
@@ -95,189 +132,137 @@ __global__ void __launch_bounds__(256) k_bc_count(int64_t n, const int32_t* __re
     }
 }
 
-// kept entries keep their order; nidx == NULL refills values only; U: the
-// type of the filtered values (an FP32 copy of an FP64 matrix is rounded once)
-template <class T, class U>
-__global__ void __launch_bounds__(256) k_bc_fill(int64_t n, const int32_t* __restrict__ indptr,
-                                                const int32_t* __restrict__ indices, const T* __restrict__ vals,
+// The Dirichlet condition on a CSR matrix.  VAL 1: the filtered matrix (a unit
+// row on boundary rows, boundary columns left out; kept entries keep their
+// order); VAL 2: the values on A's own pattern (boundary rows 1 on the diagonal
+// and 0 elsewhere, boundary columns 0; nval may be vals itself: a chunk is read
+// before any of it is written); VAL 0: none.  RHS: out = f - A uh, uh on
+// boundary rows, summed in one order whatever VAL.  As in k_spmv a block streams the contiguous entries of 256 / G rows;
+// the kept ones' new places are contiguous too: the first row's, plus the kept
+// entries before (ballots, a prefix over the block's waves), so values leave
+// in order.  Of a boundary row the first entry keeps a place, for the row's
+// thread to fill; a boundary row without entries has none, and the block that
+// sees its count fall short places its rows one by one.  nidx == NULL refills
+// values only; U: the type of the filtered values (an FP32 copy of an FP64
+// matrix is rounded once).  Both directions of HBM bound it: 20 bytes an entry.
+// 15.0M entries (100 x 113 x 90 cells, P1): 16 lanes a row 128 -> 75 us.
+template <class T, class U, int G, int VAL, bool RHS>
+__global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __restrict__ indptr,
+                                                const int32_t* __restrict__ indices, const T* vals,
                                                 const uint8_t* __restrict__ bd, const int32_t* __restrict__ nptr,
-                                                int32_t* __restrict__ nidx, U* __restrict__ nval) {
-    // two of a group's rows at a time, every load of a row issued before any
-    // of its results is needed (row bounds with the boundary flag, values
-    // with the column indices): three rounds of loads per pair of rows
-    constexpr int R = 2;
-    const int lane = threadIdx.x % BCG;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x / BCG;
-    for (int64_t r0 = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / BCG; r0 < n; r0 += R * stride) {
-        // row data of both rows (a row past n reads row n - 1 and is skipped
-        // below): all loads issued, then used
-        int32_t o0[R], k0[R], k1[R];
-        bool rb[R];
+                                                int32_t* __restrict__ nidx, U* nval,
+                                                const T* __restrict__ uh, const T* __restrict__ f,
+                                                T* __restrict__ out) {
+    constexpr int RB = 256 / G, CH = STREAM / 2, PER = CH / 256, WAVES = 256 / WAVE;
+    __shared__ T prod[RHS ? CH : 1];
+    __shared__ uint8_t mark[CH];  // 1: entry of a boundary row, 2: its first
+    __shared__ int cnt[PER * WAVES];
+    const int lane = threadIdx.x % G, wave = threadIdx.x / WAVE;
+    const unsigned long long below = (1ull << (threadIdx.x % WAVE)) - 1;
+    for (int64_t r0 = (int64_t)xcd_window_block() * RB; r0 < n; r0 += (int64_t)gridDim.x * RB) {
+        const int64_t end = min(r0 + RB, n), r = min(r0 + threadIdx.x / G, end);
+        const int32_t e0 = indptr[r0], e1 = indptr[end];
+        const int32_t k0 = indptr[r], k1 = indptr[min(r + 1, end)];
+        const int32_t o0 = VAL == 1 ? nptr[r0] : 0, o1 = VAL == 1 ? nptr[end] : 0;
+        const bool fixed = r < end && bd[r] != 0;
+        int32_t at = o0;
+        T s = T(0);
+        for (int32_t e = e0; e < e1; e += CH) {
+            const int m = min(CH, e1 - e);
+            reinterpret_cast<uint32_t*>(mark)[threadIdx.x] = 0;
+            int32_t c[PER];
+            T v[PER], w[PER];
+            bool cb[PER];
 #pragma unroll
-        for (int u = 0; u < R; ++u) {
-            const int64_t r = min(r0 + u * stride, n - 1);
-            o0[u] = nptr[r];
-            rb[u] = bd[r] != 0;
-            k0[u] = indptr[r];
-            k1[u] = indptr[r + 1];
-        }
-        // the first BCG entries of both rows: column indices and values, then
-        // the columns' boundary flags, all loads issued before the results
-        // are used (positions clamped into the row; none for an empty row)
-        int32_t c[R];
-        T v[R];
-        bool all = true;
-#pragma unroll
-        for (int u = 0; u < R; ++u) all = all && k1[u] > k0[u];
-        if (all) {  // the usual case: no empty row, the loads in one straight run
-#pragma unroll
-            for (int u = 0; u < R; ++u) {
-                const int32_t k = k0[u] + min(lane, k1[u] - k0[u] - 1);
+            for (int u = 0; u < PER; ++u) {
+                const int32_t k = e + min(u * 256 + (int)threadIdx.x, m - 1);
                 c[u] = indices[k];
                 v[u] = vals[k];
             }
-        } else {
+            __syncthreads();
+            if (fixed)
+                for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) mark[k - e] = k == k0 ? 2 : 1;
 #pragma unroll
-            for (int u = 0; u < R; ++u) {
-                const int32_t k = k0[u] + min(lane, k1[u] - k0[u] - 1);
-                c[u] = 0;
-                v[u] = T(0);
-                if (k1[u] > k0[u]) {
-                    c[u] = indices[k];
-                    v[u] = vals[k];
+            for (int u = 0; u < PER; ++u) {
+                cb[u] = bd[c[u]] != 0;
+                if constexpr (RHS) w[u] = uh[c[u]];
+            }
+            __syncthreads();
+            if constexpr (VAL == 2) {
+                if (fixed)
+                    for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G)
+                        nval[k] = indices[k] == r ? U(1) : U(0);
+            }
+            bool keep[PER];
+            int rank[PER];
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int i = u * 256 + threadIdx.x;
+                const int mk = i < m ? mark[i] : 1;
+                if constexpr (VAL == 1) {
+                    const bool place = mk == 2 || (mk == 0 && !cb[u]);
+                    keep[u] = mk == 0 && place;
+                    const unsigned long long b = __ballot(place);
+                    rank[u] = __popcll(b & below);
+                    if (threadIdx.x % WAVE == 0) cnt[u * WAVES + wave] = __popcll(b);
+                }
+                if constexpr (VAL == 2) {
+                    if (mk == 0) nval[e + i] = cb[u] ? U(0) : static_cast<U>(v[u]);
+                }
+                if constexpr (RHS) {
+                    if (i < m) prod[i] = v[u] * w[u];
                 }
             }
-        }
-        bool cb[R];
+            __syncthreads();
+            if constexpr (VAL == 1) {
 #pragma unroll
-        for (int u = 0; u < R; ++u) cb[u] = bd[c[u]] != 0;
+                for (int u = 0; u < PER; ++u)
 #pragma unroll
-        for (int u = 0; u < R; ++u) {
-            const int64_t r = r0 + u * stride;
-            if (r >= n) break;  // the same for the group's lanes
-            if (rb[u]) {
-                if (lane == 0) {
-                    if (nidx) nidx[o0[u]] = static_cast<int32_t>(r);
-                    nval[o0[u]] = U(1);
-                }
-                continue;
-            }
-            int32_t base = o0[u];
-            for (int32_t kb = k0[u]; kb < k1[u]; kb += BCG) {
-                const int32_t k = kb + lane;
-                int32_t cc = c[u];
-                T vv = v[u];
-                bool keep = false;
-                if (k < k1[u]) {
-                    if (kb != k0[u]) {  // entries past the first BCG: loaded here
-                        cc = indices[k];
-                        vv = vals[k];
-                        keep = !bd[cc];
-                    } else {
-                        keep = !cb[u];
+                    for (int q = 0; q < WAVES; ++q) {
+                        if (q == wave && keep[u] && at + rank[u] < o1) {
+                            if (nidx) nidx[at + rank[u]] = c[u];
+                            nval[at + rank[u]] = static_cast<U>(v[u]);
+                        }
+                        at += cnt[u * WAVES + q];
                     }
-                }
-                const int inc = group_inclusive_scan<BCG>(keep ? 1 : 0);
-                if (keep) {
-                    if (nidx) nidx[base + inc - 1] = cc;
-                    nval[base + inc - 1] = static_cast<U>(vv);
-                }
-                base += __shfl(inc, BCG - 1, BCG);  // group total
             }
+            if constexpr (RHS)
+                for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s += prod[k - e];
+            __syncthreads();
+        }
+        if (at != o1) {  // a boundary row without entries, the same for the whole block
+            if (lane == 0 && r < end && !fixed) {
+                int32_t o = nptr[r];
+                for (int32_t k = k0; k < k1; ++k)
+                    if (!bd[indices[k]]) {
+                        if (nidx) nidx[o] = indices[k];
+                        nval[o++] = static_cast<U>(vals[k]);
+                    }
+            }
+            __syncthreads();
+        }
+        if constexpr (RHS) s = group_sum<G>(s);
+        if (lane == 0 && r < end) {
+            if (VAL == 1 && fixed) {
+                const int32_t o = nptr[r];
+                if (nidx) nidx[o] = static_cast<int32_t>(r);
+                nval[o] = U(1);
+            }
+            if constexpr (RHS) out[r] = fixed ? uh[r] : f[r] - s;
         }
     }
 }
 
-template <class T>
-__global__ void __launch_bounds__(256) k_bc_rhs(int64_t n, const int32_t* __restrict__ indptr,
-                                               const int32_t* __restrict__ indices, const T* __restrict__ vals,
-                                               const uint8_t* __restrict__ bd, const T* __restrict__ uh,
-                                               const T* __restrict__ f, T* __restrict__ out) {
-    const int lane = threadIdx.x % BCG;
-    for (int64_t r = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / BCG; r < n;
-         r += (int64_t)gridDim.x * blockDim.x / BCG) {
-        T s = T(0);
-        if (!bd[r])
-            for (int32_t k = indptr[r] + lane; k < indptr[r + 1]; k += BCG) s += vals[k] * uh[indices[k]];
-        s = group_sum<BCG>(s);
-        if (lane == 0) out[r] = bd[r] ? uh[r] : f[r] - s;
-    }
-}
-
-// k_bc_fill (values only) and k_bc_rhs in one pass over A: the same lane
-// order for both, so the filtered values and f - A g equal the two separate
-// kernels' bit for bit
-template <class T>
-__global__ void __launch_bounds__(256) k_bc_apply(int64_t n, const int32_t* __restrict__ indptr,
-                                                 const int32_t* __restrict__ indices, const T* __restrict__ vals,
-                                                 const uint8_t* __restrict__ bd, const int32_t* __restrict__ nptr,
-                                                 T* __restrict__ nval, const T* __restrict__ uh,
-                                                 const T* __restrict__ f, T* __restrict__ out) {
-    const int lane = threadIdx.x % BCG;
-    for (int64_t r = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / BCG; r < n;
-         r += (int64_t)gridDim.x * blockDim.x / BCG) {
-        const int32_t o0 = nptr[r];
-        if (bd[r]) {
-            if (lane == 0) {
-                nval[o0] = T(1);
-                out[r] = uh[r];
-            }
-            continue;
-        }
-        int32_t base = o0;
-        T acc = T(0);
-        const int32_t k1 = indptr[r + 1];
-        for (int32_t k0 = indptr[r]; k0 < k1; k0 += BCG) {
-            const int32_t k = k0 + lane;
-            bool keep = false;
-            T v = T(0);
-            if (k < k1) {
-                const int32_t c = indices[k];
-                v = vals[k];
-                acc += v * uh[c];
-                keep = !bd[c];
-            }
-            const int inc = group_inclusive_scan<BCG>(keep ? 1 : 0);
-            if (keep) nval[base + inc - 1] = v;
-            base += __shfl(inc, BCG - 1, BCG);
-        }
-        acc = group_sum<BCG>(acc);
-        if (lane == 0) out[r] = f[r] - acc;
-    }
-}
-
-// Pattern-preserving form of k_bc_apply: the values stay on A's pattern, a
-// boundary row becomes the unit row (1 on the diagonal, 0 elsewhere) and a
-// boundary column of an interior row becomes 0; f - A g is formed in the same
-// lane order as k_bc_apply, so it equals that kernel's bit for bit.  Each
-// entry is read and written by the same lane, so nval may be vals itself.
-template <class T>
-__global__ void __launch_bounds__(256) k_bc_keep(int64_t n, const int32_t* __restrict__ indptr,
-                                                const int32_t* __restrict__ indices, const T* vals,
-                                                const uint8_t* __restrict__ bd, T* nval, const T* __restrict__ uh,
-                                                const T* __restrict__ f, T* __restrict__ out) {
-    const int lane = threadIdx.x % BCG;
-    for (int64_t r = (blockIdx.x * (int64_t)blockDim.x + threadIdx.x) / BCG; r < n;
-         r += (int64_t)gridDim.x * blockDim.x / BCG) {
-        const int32_t k1 = indptr[r + 1];
-        if (bd[r]) {
-            for (int32_t k = indptr[r] + lane; k < k1; k += BCG) nval[k] = indices[k] == r ? T(1) : T(0);
-            if (lane == 0) out[r] = uh[r];
-            continue;
-        }
-        T acc = T(0);
-        for (int32_t k0 = indptr[r]; k0 < k1; k0 += BCG) {
-            const int32_t k = k0 + lane;
-            if (k < k1) {
-                const int32_t c = indices[k];
-                const T v = vals[k];
-                acc += v * uh[c];
-                nval[k] = bd[c] ? T(0) : v;
-            }
-        }
-        acc = group_sum<BCG>(acc);
-        if (lane == 0) out[r] = f[r] - acc;
-    }
+template <class T, class U, int VAL, bool RHS>
+static int bc_launch(int64_t n, const int32_t* indptr, const int32_t* indices, const void* vals, const uint8_t* bd,
+                     const int32_t* nptr, int32_t* nidx, void* nval, const void* uh, const void* f, void* out,
+                     hipStream_t s) {
+    constexpr int G = 4;  // 64 rows a block: 960 entries of a P1 tetrahedral matrix, a chunk
+    hipLaunchKernelGGL((k_bc_rows<T, U, G, VAL, RHS>), dim3(xcd_window_grid(grid_for(n * G, 256, 1 << 20))), dim3(256), 0, s,
+                       n, indptr, indices, static_cast<const T*>(vals), bd, nptr, nidx, static_cast<U*>(nval),
+                       static_cast<const T*>(uh), static_cast<const T*>(f), static_cast<T*>(out));
+    FA_LAUNCH("k_bc_rows");
+    return FA_OK;
 }
 
 // ---- vector kernels --------------------------------------------------------------
@@ -385,21 +370,11 @@ extern "C" int fa_dirichlet_fill(int dtype, int dtype_out, int64_t n, const int3
     FA_REQUIRE(dtype_out == dtype || (dtype == FA_F64 && dtype_out == FA_F32),
                "fa_dirichlet_fill: values of dtype %d cannot be stored as dtype %d", dtype, dtype_out);
     hipStream_t s = S(stream);
-    const unsigned grid = grid_for(n * BCG, 256, 1 << 16);
-    if (dtype == FA_F64 && dtype_out == FA_F64)
-        hipLaunchKernelGGL((k_bc_fill<double, double>), dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const double*>(values), is_bd, new_indptr, new_indices,
-                           static_cast<double*>(new_values));
-    else if (dtype == FA_F64)
-        hipLaunchKernelGGL((k_bc_fill<double, float>), dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const double*>(values), is_bd, new_indptr, new_indices,
-                           static_cast<float*>(new_values));
-    else
-        hipLaunchKernelGGL((k_bc_fill<float, float>), dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const float*>(values), is_bd, new_indptr, new_indices,
-                           static_cast<float*>(new_values));
-    FA_LAUNCH("k_bc_fill");
-    return FA_OK;
+    if (n == 0) return FA_OK;
+    auto fill = dtype == FA_F32       ? bc_launch<float, float, 1, false>
+                : dtype_out == FA_F64 ? bc_launch<double, double, 1, false>
+                                      : bc_launch<double, float, 1, false>;
+    return fill(n, indptr, indices, values, is_bd, new_indptr, new_indices, new_values, nullptr, nullptr, nullptr, s);
 }
 
 extern "C" int fa_dirichlet_rhs(int dtype, int64_t n, const int32_t* indptr, const int32_t* indices,
@@ -407,17 +382,9 @@ extern "C" int fa_dirichlet_rhs(int dtype, int64_t n, const int32_t* indptr, con
                                 fa_stream_t stream) {
     FA_REQUIRE(dtype == FA_F64 || dtype == FA_F32, "fa_dirichlet_rhs: bad dtype %d", dtype);
     hipStream_t s = S(stream);
-    const unsigned grid = grid_for(n * BCG, 256, 1 << 16);
-    if (dtype == FA_F64)
-        hipLaunchKernelGGL(k_bc_rhs<double>, dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const double*>(values), is_bd, static_cast<const double*>(uh),
-                           static_cast<const double*>(f), static_cast<double*>(f_out));
-    else
-        hipLaunchKernelGGL(k_bc_rhs<float>, dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const float*>(values), is_bd, static_cast<const float*>(uh),
-                           static_cast<const float*>(f), static_cast<float*>(f_out));
-    FA_LAUNCH("k_bc_rhs");
-    return FA_OK;
+    if (n == 0) return FA_OK;
+    auto rhs = dtype == FA_F64 ? bc_launch<double, double, 0, true> : bc_launch<float, float, 0, true>;
+    return rhs(n, indptr, indices, values, is_bd, nullptr, nullptr, nullptr, uh, f, f_out, s);
 }
 
 extern "C" int fa_dirichlet_apply(int dtype, int64_t n, const int32_t* indptr, const int32_t* indices,
@@ -425,19 +392,12 @@ extern "C" int fa_dirichlet_apply(int dtype, int64_t n, const int32_t* indptr, c
                                   void* new_values, const void* uh, const void* f, void* f_out, fa_stream_t stream) {
     FA_REQUIRE(dtype == FA_F64 || dtype == FA_F32, "fa_dirichlet_apply: bad dtype %d", dtype);
     hipStream_t s = S(stream);
-    const unsigned grid = grid_for(n * BCG, 256, 1 << 16);
+    if (n == 0) return FA_OK;
     timer_begin(FA_TIMER_BC_APPLY, s);
-    if (dtype == FA_F64)
-        hipLaunchKernelGGL(k_bc_apply<double>, dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const double*>(values), is_bd, new_indptr, static_cast<double*>(new_values),
-                           static_cast<const double*>(uh), static_cast<const double*>(f), static_cast<double*>(f_out));
-    else
-        hipLaunchKernelGGL(k_bc_apply<float>, dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const float*>(values), is_bd, new_indptr, static_cast<float*>(new_values),
-                           static_cast<const float*>(uh), static_cast<const float*>(f), static_cast<float*>(f_out));
+    auto apply = dtype == FA_F64 ? bc_launch<double, double, 1, true> : bc_launch<float, float, 1, true>;
+    const int st = apply(n, indptr, indices, values, is_bd, new_indptr, nullptr, new_values, uh, f, f_out, s);
     timer_end(FA_TIMER_BC_APPLY, s);
-    FA_LAUNCH("k_bc_apply");
-    return FA_OK;
+    return st;
 }
 
 extern "C" size_t fa_reduce_work_bytes(void) { return 3 * align_up(RED_GRID * sizeof(double)) + 1024; }
@@ -632,17 +592,9 @@ extern "C" int fa_dirichlet_apply_keep(int dtype, int64_t n, const int32_t* indp
                "fa_dirichlet_apply_keep: bad arguments");
     if (n == 0) return FA_OK;
     hipStream_t s = S(stream);
-    const unsigned grid = grid_for(n * BCG, 256, 1 << 16);
     timer_begin(FA_TIMER_BC_APPLY, s);
-    if (dtype == FA_F64)
-        hipLaunchKernelGGL(k_bc_keep<double>, dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const double*>(values), is_bd, static_cast<double*>(new_values),
-                           static_cast<const double*>(uh), static_cast<const double*>(f), static_cast<double*>(f_out));
-    else
-        hipLaunchKernelGGL(k_bc_keep<float>, dim3(grid), dim3(256), 0, s, n, indptr, indices,
-                           static_cast<const float*>(values), is_bd, static_cast<float*>(new_values),
-                           static_cast<const float*>(uh), static_cast<const float*>(f), static_cast<float*>(f_out));
+    auto keep = dtype == FA_F64 ? bc_launch<double, double, 2, true> : bc_launch<float, float, 2, true>;
+    const int st = keep(n, indptr, indices, values, is_bd, nullptr, nullptr, new_values, uh, f, f_out, s);
     timer_end(FA_TIMER_BC_APPLY, s);
-    FA_LAUNCH("k_bc_keep");
-    return FA_OK;
+    return st;
 }
