@@ -350,6 +350,13 @@ BOX_ASSEMBLY = True
 RECORDS_MIN_CELLS = 200_000
 
 
+# Smaller triangle meshes evaluate a separable source in the fused load-vector
+# kernel, per vertex of each cell: one call less (64^2 cells, 8 Fourier modes:
+# 78 against 89 us, host and all; 180^2: 118 against 88 us; on tetrahedra the
+# element vectors win at 8^3 already, 536 against 110 us for a six-term source).
+SEP_ONCE_MIN_CELLS = 20_000
+
+
 def _box_grid(space, pat):
     """(nx, ny, nz) when the P1 matrix can take the structured one-pass kernel:
     a TetrahedronMesh.from_box mesh (no threshold) and the space's own pattern."""
@@ -444,6 +451,14 @@ def p1_vector_values(space, it, pat, dtype):
         nat.check(L.fa_sum_incidence_values(nat.dtype_code(dtype), pat.gdof, nat.ptr(pat.adj_ptr), nat.ptr(vals),
                                             nat.ptr(out), nat.stream()), "fa_sum_incidence_values")
         return out
+    if kind == nat.COEF_SEP and (space.TD == 3 or pat.nc >= SEP_ONCE_MIN_CELLS):
+        # each point evaluated once, not once per vertex of its cell
+        elem = torch.empty((pat.nc, pat.ldof), dtype=torch.float64, device=space.device)
+        nat.check(L.fa_element_vectors(nat.FA_F64, space.TD, pat.ldof, qw.shape[0], nat.ptr(mesh.node),
+                                       nat.ptr(space.cell_to_dof()), pat.nc, nat.ptr(qw), nat.ptr(phi), kind, scale,
+                                       nat.ptr(src), nat.ptr(elem), nat.stream()), "fa_element_vectors")
+        v = pat.gather_vector(elem)
+        return v if dtype == torch.float64 else v.to(dtype)
     nat.check(L.fa_assemble_p1_vector(nat.dtype_code(dtype), space.TD, pat.gdof, qw.shape[0], nat.ptr(mesh.node),
                                       nat.ptr(space.cell_to_dof()), nat.ptr(qw), nat.ptr(phi), kind, scale,
                                       nat.ptr(src), nat.ptr(pat.adj_ptr), nat.ptr(pat.adj), nat.ptr(out),
