@@ -294,10 +294,12 @@ def rooflines(kt, mesh, gdof, nnz_a, nnz_bc, n, vb, vb_a=8):
     else:
         asm_a = _roof("k_p1_incidence_rows<3> + k_sum_incidence_rows", b_a, 1, m1 + m2,
                       pass1_us=round(m1 * 1e3 / max(l1, 1), 2), pass2_us=round(m2 * 1e3 / max(l2, 1), 2))
-    fname = ("k_p1_box_cell_vectors + k_p1_box_sum_vectors" if lb else
+    one_pass = lb and not l4        # a separable source on a tensor grid
+    fname = ("k_p1_box_vector" if one_pass else "k_p1_box_cell_vectors + k_p1_box_sum_vectors" if lb else
              "k_p1_incidence_vectors<3> + k_sum_incidence_values")
     # the structured kernels read no cell array: coordinates, k, the vector out
-    asm_f = _roof(fname, 24 * nn + 8 * nc + 8 * gdof if lb else b_f, 1, m3 + m4, BOX_F_TRAFFIC_128 if (big and lb) else None,
+    asm_f = _roof(fname, 24 * nn + 8 * nc + 8 * gdof if lb else b_f, 1, m3 + m4,
+                  BOX_F_TRAFFIC_128 if (big and lb and not one_pass) else None,
                   pass1_us=round(m3 * 1e3 / max(l3, 1), 2), pass2_us=round(m4 * 1e3 / max(l4, 1), 2))
     vl, vms = kt["vcycle"]
     dl, dms = kt["dirichlet"]
