@@ -20,12 +20,14 @@ def _check_tensor_space(space, who):
 
 def _precontracted(space, q):
     """M[i, j, m, n] = sum_q w_q R[q, i, m] R[q, j, n] (FP64, on the device),
-    cached per quadrature index."""
+    cached per quadrature index, complete before another stream or thread can see it."""
     ss = space.scalar_space
     cache = ss.__dict__.setdefault('_elast_M', {})
     if q not in cache:
         _, qw, _, R = ss.tables(q)                                   # R: (NQ, ldof, TD+1)
-        cache[q] = torch.einsum('q, qim, qjn -> ijmn', qw, R, R).contiguous()
+        M = torch.einsum('q, qim, qjn -> ijmn', qw, R, R).contiguous()
+        torch.cuda.current_stream(M.device).synchronize()
+        cache[q] = M
     return cache[q]
 
 

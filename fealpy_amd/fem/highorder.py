@@ -57,6 +57,7 @@ def mfma_tables(space, q, precision):
     groups = math.ceil(ntiles / tpg)
     btab = fragment_order(K, ks, per_lane, tpg, groups)
     btab = btab.to(torch.bfloat16 if prec == 0 else torch.float32).contiguous()
+    torch.cuda.current_stream(btab.device).synchronize()         # complete before another stream or thread reads it
     cache[key] = (btab, ks, tpg, groups)
     return cache[key]
 

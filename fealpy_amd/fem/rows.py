@@ -3,28 +3,49 @@ fa_assemble_elasticity_rows) on a space's own pattern: P1 diffusion and mass
 with coefficients constant on each cell, and isotropic elasticity of any
 degree.  No array of element matrices is formed (the reference's
 ``integrator.assembly`` -> COO -> coalesce, fem/bilinear_form.py:46-105)."""
+import functools
+
+import numpy as np
 import torch
 
 from .. import _native as nat
+from ..functionspace.basis import grad_shape_function, shape_function
 from .pattern import pattern_of
 
 _PAIRS = {2: ((0, 0), (0, 1), (1, 1)), 3: ((0, 0), (0, 1), (0, 2), (1, 1), (1, 2), (2, 2))}
 
 
-def _reduced(space, q):
-    _, qw, phi, gphi = space.tables(q)
-    return qw, phi, gphi[:, :, 1:] - gphi[:, :, :1]              # sum_m grad lambda_m = 0
+@functools.lru_cache(maxsize=64)
+def _reference_sums(p, bcs, ws):
+    """(M (TD, TD, ldof, ldof), sum_q w_q phi_i phi_j) of the degree-p basis at
+    the rule (points and weights as tuples of numbers), with
+    M[a, b, i, j] = sum_q w_q R'_ia R'_jb, R' the reference gradients reduced by
+    sum_m grad lambda_m = 0.  Formed on the host, so that a table is complete
+    when it is uploaded, whichever stream or thread reads it first, and summed
+    in extended precision: every cell multiplies the same table, whose rounding
+    would not average out over the cells of a row."""
+    bc, w = np.array(bcs), np.array(ws, dtype=np.longdouble)
+    R = grad_shape_function(bc, p).astype(np.longdouble)
+    R = (R[:, :, 1:] - R[:, :, :1]).transpose(0, 2, 1)                # (NQ, TD, ldof)
+    phi = shape_function(bc, p).astype(np.longdouble)
+    nq, td, ldof = R.shape
+    F = np.ascontiguousarray(R).reshape(nq, -1)
+    M = ((F * w[:, None]).T @ F).reshape(td, ldof, td, ldof).transpose(0, 2, 1, 3)
+    return np.ascontiguousarray(M, dtype=np.float64), ((phi * w[:, None]).T @ phi).astype(np.float64)
+
+
+def _sums(space, q):
+    bcs, ws = space.mesh.quadrature_formula(q).get_quadrature_points_and_weights()
+    return _reference_sums(space.p, tuple(map(tuple, bcs.tolist())), tuple(ws.tolist()))
 
 
 def p1_table(space, q):
     """(NS + 1, TD + 1, TD + 1) table of fa_assemble_p1_rows, FP64, kept per rule."""
     cache = space.__dict__.setdefault('_row_tables', {})
     if q not in cache:
-        qw, phi, R = _reduced(space, q)
-        M = torch.einsum('q, qia, qjb -> abij', qw, R, R)
+        M, mass = _sums(space, q)
         rows = [M[a, b] if a == b else M[a, b] + M[b, a] for a, b in _PAIRS[space.TD]]
-        rows.append(torch.einsum('q, qi, qj -> ij', qw, phi, phi))
-        cache[q] = torch.stack(rows).contiguous()
+        cache[q] = torch.as_tensor(np.stack(rows + [mass]), device=space.device)
     return cache[q]
 
 
@@ -32,8 +53,7 @@ def elasticity_table(scalar_space, q):
     """(TD, TD, ldof, ldof) table of fa_assemble_elasticity_rows, kept per rule."""
     cache = scalar_space.__dict__.setdefault('_elast_row_tables', {})
     if q not in cache:
-        qw, _, R = _reduced(scalar_space, q)
-        cache[q] = torch.einsum('q, qia, qjb -> abij', qw, R, R).contiguous()
+        cache[q] = torch.as_tensor(_sums(scalar_space, q)[0], device=scalar_space.device)
     return cache[q]
 
 

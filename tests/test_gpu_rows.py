@@ -4,6 +4,8 @@ summed in FP64 on the CPU: meshes with shuffled numbering, a vertex of high
 degree, the smallest meshes, both value types and DOF layouts.  An entry adds at
 most `deg` cells' values, each a sum of at most 9 products on either side:
 9 deg units in the last place of the largest entry."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -85,3 +87,36 @@ def test_elasticity_rows(name, p, prio, dtype, monkeypatch):
     assert rows.elasticity_values(space, it, dtype) is not None
     A = fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype)
     _check(A, space, it.assembly(space), dtype)
+
+
+@pytest.mark.parametrize("vector", [False, True])
+def test_first_assembly_from_two_streams(vector, monkeypatch):
+    """Two threads, a stream each, assemble on a space whose tables and row positions neither has built yet."""
+    monkeypatch.setattr(integrators, "RECORDS_MIN_CELLS", 0)
+    monkeypatch.setattr(rows, "ELASTICITY_MIN_DOFS", 0)
+    mesh = MESHES["tet"]()
+    mat = fa.LinearElasticMaterial("m", lame_lambda=1.3, shear_modulus=0.7)
+
+    def assembled(space):
+        if vector:
+            space = fa.TensorFunctionSpace(space, (-1, 3))
+            return fa.BilinearForm(space).add_integrator(fa.LinearElasticityIntegrator(mat, q=4)).assembly().values
+        return fa.BilinearForm(space).add_integrator(fa.ScalarDiffusionIntegrator(2.0, q=3)).assembly().values
+
+    ref = assembled(fa.LagrangeFESpace(mesh, 2 if vector else 1))
+    for _ in range(4):
+        space, out, start = fa.LagrangeFESpace(mesh, 2 if vector else 1), [None, None], threading.Barrier(2)
+        torch.cuda.synchronize()
+
+        def work(i):
+            with torch.cuda.stream(torch.cuda.Stream()):
+                start.wait()
+                out[i] = assembled(space)
+                torch.cuda.current_stream().synchronize()
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert torch.equal(out[0], ref) and torch.equal(out[1], ref)
