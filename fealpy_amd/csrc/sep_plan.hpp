@@ -47,7 +47,8 @@ __device__ inline void sep_plan(const fa_sep_t* __restrict__ e, SepPlan& p) {
     for (int j = nf - 1; j >= 0; --j) {
         const int cj = __shfl(cls, j), dj = __shfl(dim, j), oj = __shfl(cosine, j);
         const double aj = __shfl(a, j), bj = __shfl(b, j);
-        if (cj == cls && dj == dim && aj == a && bj == b) {
+        // a factor matches itself whatever its numbers: a NaN equals nothing
+        if (j == k || (cj == cls && dj == dim && aj == a && bj == b)) {
             if (j < k) first = j;
             us |= !oj;
             uc |= oj;

@@ -16,6 +16,7 @@ from fealpy_amd.functionspace.basis import shape_function
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
+NAN = float("nan")
 PI = math.pi
 
 
@@ -79,3 +80,24 @@ def test_sampled_source_and_its_sum(dtype):
     got = fa.LinearForm(space).add_integrator(fa.ScalarSourceIntegrator(f.to(DEV), q=5)).assembly(dtype=dtype).cpu()
     eps = 2.2e-16 if dtype == torch.float64 else 1.2e-7 / 35     # one rounding of each element value and add
     assert float((got.double() - full).abs().max()) <= 2 * 35 * eps * float(full.abs().max())
+
+
+@pytest.mark.parametrize("factor", [lambda s, a, b: expr.sin(a * s + b), lambda s, a, b: expr.cos(a * s + b),
+                                    lambda s, a, b: expr.exp(a * s + b), lambda s, a, b: a * s + b])
+@pytest.mark.parametrize("a,b", [(NAN, 0.5), (2.0, NAN), (NAN, NAN)])
+def test_nan_parameters(factor, a, b):
+    """A factor with a NaN in it makes its term NaN at every point, beside terms of other factors, and reaches
+    nothing else: the same forms without it are as they were."""
+    mesh = fa.TriangleMesh.from_box(nx=9, ny=8, device=DEV)
+    space = fa.LagrangeFESpace(mesh, 2)
+    other = 1.0 + expr.exp(expr.x) * expr.sin(2.0 * expr.y) + expr.cos(expr.x) * (expr.y + 2.0)
+
+    def forms(f):
+        return (fa.LinearForm(space).add_integrator(fa.ScalarSourceIntegrator(f, q=4)).assembly(),
+                fa.BilinearForm(space).add_integrator(fa.ScalarDiffusionIntegrator(f, q=4)).assembly().values)
+
+    before = forms(other)
+    for out in forms(other + factor(expr.x, a, b) * expr.cos(expr.y)):
+        assert bool(torch.isnan(out).all())
+    for out, ref in zip(forms(other), before):
+        assert torch.equal(out, ref) and bool(torch.isfinite(out).all())
