@@ -132,8 +132,9 @@ __device__ inline void lds_add(double* p, double v) {
     __hip_atomic_fetch_add(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// ldof lanes per row, 64 / ldof rows per wave (one, and ldof / 64 rounds, past
-// 64); a row's FP64 sums live in LDS.  Lane j adds entry (i, j) of the row's
+// ldof lanes per row, up to 64 / ldof rows per wave (one, and ldof / 64 rounds,
+// past 64; fewer where the longest row's sums would not fit otherwise); a row's
+// FP64 sums live in LDS.  Lane j adds entry (i, j) of the row's
 // incident cells in ascending order, which is the order of the reference's
 // stable lexsort + sequential np.add.at.  The additions of one wave to LDS are
 // done in the order it issues them, so they are LDS adds without a result
@@ -146,14 +147,14 @@ __device__ inline void lds_add(double* p, double v) {
 constexpr int SUM_U = 4;
 
 template <int LDOF, class T>
-__global__ void __launch_bounds__(256) k_sum_rows(int64_t gdof, int ld, const int32_t* __restrict__ ptr,
+__global__ void __launch_bounds__(256) k_sum_rows(int64_t gdof, int ld, int rows, const int32_t* __restrict__ ptr,
                                                   const int32_t* __restrict__ adj, const int32_t* __restrict__ indptr,
                                                   const uint16_t* __restrict__ pos, int lmax,
                                                   const T* __restrict__ elem, int64_t cpad, T* __restrict__ values) {
     extern __shared__ double sums[];
     const int ldof = LDOF ? LDOF : ld;  // LDOF 0: any width, known at run time
     const int lane = threadIdx.x % WAVE, wave = threadIdx.x / WAVE;
-    const int width = min(ldof, WAVE), rows = WAVE / width;
+    const int width = min(ldof, WAVE);
     const int sub = lane / width, j0 = lane - sub * width;
     double* acc = sums + (wave * rows + min(sub, rows - 1)) * lmax;
     const int64_t per_block = (int64_t)(blockDim.x / WAVE) * rows;
@@ -198,7 +199,10 @@ __global__ void __launch_bounds__(256) k_sum_rows(int64_t gdof, int ld, const in
 template <int LDOF, class T>
 static int launch_sum_rows(int64_t gdof, int ldof, const int32_t* ptr, const int32_t* adj, const int32_t* indptr,
                            const uint16_t* pos, int lmax, const void* elem, int64_t cpad, void* values, hipStream_t s) {
-    const int rows = WAVE / std::min(ldof, WAVE);
+    // a wave's sums take 64 KB at most: every row that a pattern can hold (8192
+    // entries) fits, and two waves share a CU beside one long row
+    int rows = WAVE / std::min(ldof, WAVE);
+    while (rows > 1 && sizeof(double) * rows * lmax > 64 * 1024) rows >>= 1;
     const size_t per_wave = sizeof(double) * rows * lmax;
     int waves = 4;
     while (waves > 1 && waves * per_wave > 32 * 1024) waves >>= 1;
@@ -212,7 +216,7 @@ static int launch_sum_rows(int64_t gdof, int ldof, const int32_t* ptr, const int
         FA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
                                    static_cast<int>(lds)));
     const unsigned grid = xcd_window_grid(static_cast<unsigned>((gdof + waves * rows - 1) / (waves * rows)));
-    hipLaunchKernelGGL(k, dim3(grid), dim3(waves * WAVE), lds, s, gdof, ldof, ptr, adj, indptr, pos, lmax,
+    hipLaunchKernelGGL(k, dim3(grid), dim3(waves * WAVE), lds, s, gdof, ldof, rows, ptr, adj, indptr, pos, lmax,
                        static_cast<const T*>(elem), cpad, static_cast<T*>(values));
     FA_LAUNCH("k_sum_rows");
     return FA_OK;

@@ -120,3 +120,14 @@ def test_first_assembly_from_two_streams(vector, monkeypatch):
         for t in threads:
             t.join()
         assert torch.equal(out[0], ref) and torch.equal(out[1], ref)
+
+
+@pytest.mark.parametrize("p,n", [(1, 980), (1, 2700), (2, 700), (2, 1300)])
+def test_long_rows_sum_from_elements(p, n):
+    """One vertex of very many triangles: rows longer than 64 / ldof of them would fit in LDS."""
+    fan = _fan(n)
+    cell = (fan.cell + n) % (n + 1)          # the centre last: the edge builder takes 1024 edges from their smallest vertex
+    space = fa.LagrangeFESpace(fa.TriangleMesh(fan.node.roll(-1, 0).contiguous(), cell.to(torch.int32)), p)
+    it = fa.ScalarDiffusionIntegrator(2.0, q=p + 1)
+    for dtype in (torch.float64, torch.float32):
+        _check(fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype), space, it.assembly(space), dtype)
