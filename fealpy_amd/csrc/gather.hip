@@ -166,9 +166,9 @@ __global__ void __launch_bounds__(256) k_sum_rows(int64_t gdof, int ld, int rows
     for (int t = j0; t < L; t += width) acc[t] = 0.0;
     wave_lds_fence();
     const int32_t* ad = adj + k0;
-    for (int j = j0; j < ldof; j += width) {
-        const uint16_t* pr = pos + (int64_t)k0 * ldof + j;
-        const T* el = elem + j;
+    if (ldof <= WAVE) {
+        const uint16_t* pr = pos + (int64_t)k0 * ldof + j0;
+        const T* el = elem + j0;
         for (int k = 0; k < deg; k += SUM_U) {
             // straight-line loads (the last incidence again past the end): a
             // test around each would wait for one before issuing the next
@@ -190,6 +190,22 @@ __global__ void __launch_bounds__(256) k_sum_rows(int64_t gdof, int ld, int rows
 #pragma unroll
             for (int u = 0; u < SUM_U; ++u)
                 if (k + u < deg) lds_add(acc + p[u], v[u]);
+        }
+    } else {
+        // all rounds of one incidence before the next incidence's: with the
+        // rounds outermost an entry met in two of them would not be summed in
+        // cell order
+        for (int k = 0; k < deg; ++k) {
+            const uint32_t e = ad[k];
+            const uint16_t* pr = pos + (int64_t)(k0 + k) * ldof;
+            const T* el = elem + (uint64_t)e * (uint32_t)ldof + e / (uint32_t)ldof * cpad;
+            for (int j = j0; j < ldof; j += 2 * WAVE) {
+                const int j1 = min(j + WAVE, ldof - 1);
+                const int p0 = pr[j], p1 = pr[j1];
+                const T v0 = el[j], v1 = el[j1];
+                lds_add(acc + p0, v0);
+                if (j + WAVE < ldof) lds_add(acc + p1, v1);
+            }
         }
     }
     wave_lds_fence();

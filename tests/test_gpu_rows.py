@@ -39,7 +39,8 @@ MESHES = {"tri1": lambda: fa.TriangleMesh.from_box(nx=1, ny=1, device=DEV),
           "tri": lambda: _shuffled(fa.TriangleMesh.from_box(nx=9, ny=7, device=DEV), 1),
           "fan": lambda: _fan(300),
           "tet1": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=1, ny=1, nz=1, device=DEV), 2),
-          "tet": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=4, ny=3, nz=5, device=DEV), 3)}
+          "tet2": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=2, ny=1, nz=2, device=DEV), 5),
+         "tet": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=4, ny=3, nz=5, device=DEV), 3)}
 
 
 def _dense(space, elem):
@@ -131,3 +132,24 @@ def test_long_rows_sum_from_elements(p, n):
     it = fa.ScalarDiffusionIntegrator(2.0, q=p + 1)
     for dtype in (torch.float64, torch.float32):
         _check(fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype), space, it.assembly(space), dtype)
+
+
+@pytest.mark.parametrize("name,p,vector", [("tri", 3, False), ("tet", 2, False), ("tri", 4, True), ("tet2", 3, True),
+                                           ("tet1", 4, True), ("tet2", 4, True)])
+def test_rows_sum_in_cell_order(name, p, vector, monkeypatch):
+    """Every entry adds its cells' values one after another in ascending cell order, also where an element row is
+    wider than a wave (105 columns): bit for bit np.add.at."""
+    mesh = MESHES[name]()
+    gd = mesh.geo_dimension()
+    space = fa.LagrangeFESpace(mesh, p)
+    it = fa.ScalarDiffusionIntegrator(2.0, q=p + 1)
+    if vector:
+        space = fa.TensorFunctionSpace(space, (-1, gd))
+        it = fa.LinearElasticityIntegrator(fa.LinearElasticMaterial("m", lame_lambda=1.3, shear_modulus=0.7,
+                                                                    **({} if gd == 3 else {"hypo": "plane_strain"})))
+        monkeypatch.setattr(rows, "elasticity_values", lambda *a: None)
+    A = fa.BilinearForm(space).add_integrator(it).assembly()
+    n, c2d = space.number_of_global_dofs(), space.cell_to_dof().cpu().numpy()
+    ref = np.zeros((n, n))
+    np.add.at(ref, (c2d[:, :, None], c2d[:, None, :]), it.assembly(space).cpu().numpy())
+    assert np.array_equal(A.to_dense().cpu().numpy(), ref)
