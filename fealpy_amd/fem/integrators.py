@@ -357,6 +357,21 @@ RECORDS_MIN_CELLS = 200_000
 SEP_ONCE_MIN_CELLS = 20_000
 
 
+# Load vectors of a separable source on a tensor grid take the one-pass kernel
+# (fa_p1_box_vector_tensor) where it keeps the factors in registers: one term at
+# the four-point rule.  A block marches several planes of cubes in sequence, and
+# any other source walks its terms point by point in each: 25^3 cells, 20 points
+# 111 us in two passes against 388 us, six terms 102 against 694, 128^3 678
+# against 2715.  Below about 32^3 cells it gains nothing (25^3: 49 against 47 us)
+# and the check of the grid lines makes the first call longer (343 against
+# 382 us; 40^3: 405 against 383; 128^3: 342 against 94 us a call).
+BOX_ONE_PASS_MIN_CELLS = 200_000
+
+
+def _box_one_pass(source, nq, nc):
+    return nc >= BOX_ONE_PASS_MIN_CELLS and nq == 4 and len(Sep.of(source).terms) == 1
+
+
 def _box_grid(space, pat):
     """(nx, ny, nz) when the P1 matrix can take the structured one-pass kernel:
     a TetrahedronMesh.from_box mesh (no threshold) and the space's own pattern."""
@@ -428,8 +443,9 @@ def p1_vector_values(space, it, pat, dtype):
         kind, scale, src = nat.COEF_CONST, 1.0, None
     out = torch.empty(pat.gdof, dtype=dtype, device=space.device)
     grid = _box_grid(space, pat)
-    axes = mesh.box_axes() if grid is not None and kind == nat.COEF_SEP else None
-    if axes is not None:         # a separable source on a tensor grid: one pass
+    one_pass = grid is not None and kind == nat.COEF_SEP and _box_one_pass(it.source, qw.shape[0], pat.nc)
+    axes = mesh.box_axes() if one_pass else None
+    if axes is not None:         # a one-term source on a tensor grid: one pass
         work = nat.workspace(L.fa_p1_box_vector_tensor_work_bytes(*grid, qw.shape[0]), space.device)
         nat.check(L.fa_p1_box_vector_tensor(nat.dtype_code(dtype), *grid, nat.ptr(mesh.node_rows16()), nat.ptr(axes),
                                             qw.shape[0], nat.ptr(qw), nat.ptr(phi), scale, nat.ptr(src), nat.ptr(out),

@@ -1,0 +1,15 @@
+"""Which kernel a call takes, where the rule can be asked without a device."""
+import pytest
+
+from fealpy_amd import expr
+from fealpy_amd.fem import integrators
+
+ONE = 2.0 * expr.sin(expr.x) * expr.cos(expr.y) * expr.exp(expr.z)
+
+
+@pytest.mark.parametrize("source,nq,n,one_pass", [
+    (ONE, 4, 128, True), (expr.x + 1.0, 4, 40, True), (ONE, 4, 25, False), (ONE, 4, 6, False), (ONE, 20, 128, False),
+    (ONE, 1, 128, False), (ONE + expr.x, 4, 128, False), (ONE + 0.5, 4, 10, False)])
+def test_one_pass_load_vector_of_a_box(source, nq, n, one_pass):
+    """Only one-term sources at the four-point rule on large grids: the others lost up to six times."""
+    assert integrators._box_one_pass(source, nq, 6 * n ** 3) is one_pass
