@@ -43,12 +43,13 @@ __global__ void __launch_bounds__(256) k_p1_box_vector(int nx, int ny, int nz, i
                                                        const fa_sep_t* __restrict__ e, const double* __restrict__ tab,
                                                        int nmax, T* __restrict__ out) {
     __shared__ double vec[24][BV_Y * BV_Z];
-    const int ly = threadIdx.x / BV_Z, lz = threadIdx.x % BV_Z;
-    const int iy = blockIdx.y * (BV_Y - 1) + ly, iz = blockIdx.x * (BV_Z - 1) + lz;  // the thread's node
+    const int ly = threadIdx.x / BV_Z, lz = threadIdx.x % BV_Z, gz = nz / (BV_Z - 1) + 1;
+    const int by = static_cast<int>(blockIdx.x) / gz, bz = static_cast<int>(blockIdx.x) - by * gz;
+    const int iy = by * (BV_Y - 1) + ly, iz = bz * (BV_Z - 1) + lz;  // the thread's node
     const int cy = iy - 1, cz = iz - 1;                                              // the thread's cube
     const bool cube = cy >= 0 && cy < ny && cz >= 0 && cz < nz;
     const bool owns = ly < BV_Y - 1 && lz < BV_Z - 1 && iy <= ny && iz <= nz;
-    const int x0 = blockIdx.z * span, x1 = min(x0 + span, nx + 1);
+    const int x0 = blockIdx.y * span, x1 = min(x0 + span, nx + 1);
     const double hy = cube ? axes[nx + 2 + cy] - axes[nx + 1 + cy] : 0.0;
     const double hz = cube ? axes[nx + ny + 3 + cz] - axes[nx + ny + 2 + cz] : 0.0;
     const int nt = e->nterms;
@@ -172,18 +173,20 @@ extern "C" int fa_p1_box_vector_tensor(int dtype, int nx, int ny, int nz, const 
     FA_REQUIRE(work_bytes >= need && (reinterpret_cast<uintptr_t>(work) & 31) == 0,
                "fa_p1_box_vector_tensor: workspace of %zu bytes (32-byte aligned) too small, %zu needed", work_bytes,
                need);
+    // tiles along one grid dimension, which takes 2^24 blocks of 256 threads: a
+    // grid with more has over 2^31 nodes or 270 GB of factor tables
+    const int64_t tiles = static_cast<int64_t>(ny / (BV_Y - 1) + 1) * (nz / (BV_Z - 1) + 1);
+    FA_REQUIRE(tiles <= (1 << 24), "fa_p1_box_vector_tensor: grid too large");
+    // about three blocks a CU, each at least four planes long
+    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((nx + 4) / 4, 3 * 256 / tiles));
+    const int span = static_cast<int>((nx + chunks) / chunks);
+    const dim3 grid(static_cast<unsigned>(tiles), static_cast<unsigned>((nx + span) / span));
     double* lines = static_cast<double*>(work);
     double* tab = reinterpret_cast<double*>(static_cast<char*>(work) + table_offset(nx, ny, nz));
     hipStream_t s = S(stream);
     timer_begin(FA_TIMER_P1_VECTORS, s);
     const int st = launch_box_sep_table(nx, ny, nz, node_wide, sep, nq, lines, tab, s);
     if (st != FA_OK) return st;
-    const unsigned gy = static_cast<unsigned>(ny / (BV_Y - 1) + 1), gz = static_cast<unsigned>(nz / (BV_Z - 1) + 1);
-    // about three blocks a CU, each at least four planes long
-    const int64_t chunks = std::max<int64_t>(1, std::min<int64_t>((nx + 4) / 4, 3 * 256 / (static_cast<int64_t>(gy) * gz)));
-    const int span = static_cast<int>((nx + chunks) / chunks);
-    const dim3 grid(gz, gy, static_cast<unsigned>((nx + span) / span));
-    FA_REQUIRE(gy <= 65535 && grid.z <= 65535, "fa_p1_box_vector_tensor: grid too large");
     const int nmax = std::max(nx, std::max(ny, nz));
     const auto* e = static_cast<const fa_sep_t*>(sep);
     if (dtype == FA_F64)

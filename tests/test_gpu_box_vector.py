@@ -42,3 +42,9 @@ def test_tensor_grid_load_vector(dims, q, name, monkeypatch):
     ref = form.assembly()
     nq = mesh.quadrature_formula(q).get_quadrature_points_and_weights()[1].shape[0]
     assert float((got - ref).abs().max()) <= (nq + 28) * 2.2e-16 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("dims", [(1, 470_000, 1), (1, 1, 470_000), (470_000, 1, 1)])
+def test_very_long_grid(dims, monkeypatch):
+    """More tiles (67,143 along y) than a grid's second dimension holds."""
+    test_tensor_grid_load_vector(dims, 1, "one", monkeypatch)
