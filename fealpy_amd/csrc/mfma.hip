@@ -13,11 +13,18 @@
 // Work split: a block takes a slice of TPG column tiles (32 ij each), whose
 // reference tensors are staged in LDS once, and a range of cells; its 4
 // wavefronts take pairs of 32-cell tiles of the range in turn.  All slices of a
-// range follow each other on one XCD, so the range's coefficients are read into
-// one L2 once and its matrices are written together; with all ranges of one
-// slice first, every slice read the coefficients again (P4, 663,552 cells, 39
-// slices: 4.1 GB beside the 3.3 GB written).  BF16 holds three waves a SIMD, one
-// operator's coefficients in registers at a time: 1.68 -> 1.51 ms there.
+// range follow each other, from MF_DEAL_RANGES ranges on each on one XCD, so the
+// range's coefficients are read into one L2 once and its matrices are written
+// together; with all ranges of one slice first, every slice read the
+// coefficients again (P4, 663,552 cells, 39 slices: 4.1 GB beside the 3.3 GB
+// written; 20^3 cells BF16 111 -> 106 us).  Fewer ranges leave XCDs idle when
+// dealt whole (P4 FP32, 3 ranges 46 against 75 us, 9 ranges 80 against 118).
+//
+// Coefficients: LATE holds one operator's at a time, diffusion's per tile, then
+// mass's; otherwise both are loaded once per pair of cell tiles.  BF16 with one
+// tile a slice (P4): LATE, three waves a SIMD, 1.68 -> 1.51 ms at 663,552 cells;
+// with two (P2, P3) it would read them per tile: 48^3 P3 0.93 against 0.56 ms,
+// P2 0.29 against 0.20 ms.  FP32: see MF_EARLY_FROM.
 #include "common.hpp"
 
 namespace fa {
@@ -27,6 +34,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int MF_CELLS_PER_BLOCK = 512;  // 16 tiles of 32 cells, 4 per wavefront
 constexpr int MF_NS = 7;                 // 6 metric components + mass
+constexpr int MF_DEAL_RANGES = 32;       // cell ranges from which a range's slices share an XCD
+// FP32 launches of MF_EARLY_FROM to MF_EARLY_TO blocks load both operators'
+// coefficients up front, others one at a time (measured, early against late, us:
+// P2 376 blocks 48/45, 732 70/73, 5184 341/338; P3 117 38/36, 429 60/65, 1222
+// 129/152, 4121 399/402, 16848 1537/1497; P4 351 84/80, 1287 200/208, 3666
+// 511/512, 12363 1667/1648)
+constexpr int MF_EARLY_FROM = 400, MF_EARLY_TO = 4608;
 
 // per-cell A operand: out[c][q] = w_q coef(c, q) (zero beyond nq), in the MFMA input type
 template <class E>
@@ -133,15 +147,15 @@ struct MfTraits<KS, false> {
 // Btab: [ngroups][MF_NS][TPG][KS][64 lanes][PER_LANE]; lane l of step ks holds
 // K_s[KSTEP*ks + PER_LANE*(l/32) + t][32*tile + l%32], t < PER_LANE.
 // A operands ad / am: (nc or 1, KS*KSTEP) rows; row stride 0 broadcasts one row.
-template <int KS, bool BF16, int TPG>
-__global__ void __launch_bounds__(256, BF16 ? 3 : 1) k_element_mfma(int64_t nc, int ldof, const double* __restrict__ node,
+template <int KS, bool BF16, int TPG, bool LATE>
+__global__ void __launch_bounds__(256, LATE && BF16 ? 3 : 1) k_element_mfma(int64_t nc, int ldof, const double* __restrict__ node,
                                                      const int32_t* __restrict__ cell,
                                                      const typename MfTraits<KS, BF16>::elem* __restrict__ ad,
                                                      int64_t ad_stride,
                                                      const typename MfTraits<KS, BF16>::elem* __restrict__ am,
                                                      int64_t am_stride,
                                                      const typename MfTraits<KS, BF16>::elem* __restrict__ btab,
-                                                     const float* __restrict__ metric, int64_t ld, int groups,
+                                                     const float* __restrict__ metric, int64_t ld, int groups, bool deal,
                                                      float* __restrict__ elem) {
     typedef MfTraits<KS, BF16> Tr;
     typedef typename Tr::elem E;
@@ -153,9 +167,9 @@ __global__ void __launch_bounds__(256, BF16 ? 3 : 1) k_element_mfma(int64_t nc, 
     float* gl = reinterpret_cast<float*>(smem + align_up(sizeof(E) * SLICE, 16));  // [4 waves][2][8][32]
     const int lane = threadIdx.x & (WAVE - 1);
     const int wave = threadIdx.x / WAVE;
-    // workgroups are dealt to the 8 XCDs in turn: range 8 k + x on XCD x, its slices one after another
-    const int nth = static_cast<int>(blockIdx.x >> 3), group = nth % groups;
-    const int64_t cbase = ((int64_t)(nth / groups) * 8 + (blockIdx.x & 7)) * MF_CELLS_PER_BLOCK;
+    // workgroups are dealt to the 8 XCDs in turn: with `deal` range 8 k + x on XCD x, its slices one after another
+    const int nth = static_cast<int>(deal ? blockIdx.x >> 3 : blockIdx.x), group = nth % groups;
+    const int64_t cbase = (deal ? (int64_t)(nth / groups) * 8 + (blockIdx.x & 7) : nth / groups) * MF_CELLS_PER_BLOCK;
     if (cbase >= nc) return;
     {   // stage the group's reference tensors (16-byte copies)
         const int4* src = reinterpret_cast<const int4*>(btab + (int64_t)group * SLICE);
@@ -171,7 +185,7 @@ __global__ void __launch_bounds__(256, BF16 ? 3 : 1) k_element_mfma(int64_t nc, 
     for (int pt = wave; pt < MF_CELLS_PER_BLOCK / 64; pt += 4) {
         const int64_t c0 = cbase + pt * 64;
         if (c0 >= nc) break;
-        F fa[2][KS];  // one operator's coefficients at a time: both would leave two waves a SIMD
+        F fa[2][KS], fm[LATE ? 1 : 2][LATE ? 1 : KS];
 #pragma unroll
         for (int h2 = 0; h2 < 2; ++h2) {
             const int64_t cl = c0 + 32 * h2 + (lane & 31);
@@ -187,15 +201,19 @@ __global__ void __launch_bounds__(256, BF16 ? 3 : 1) k_element_mfma(int64_t nc, 
                 g[(4 * h + 3) * 32 + cc] = v.w;
             }
         }
-        auto coefficients = [&](const E* a, int64_t stride) {
+        auto coefficients = [&](F (*f)[KS], const E* a, int64_t stride) {
 #pragma unroll
             for (int h2 = 0; h2 < 2; ++h2) {
                 const int64_t cl = c0 + 32 * h2 + (lane & 31), crow = cl < nc ? cl : c0;
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks)
-                    fa[h2][ks] = Tr::load(a + crow * stride + ks * Tr::KSTEP + Tr::PER_LANE * (lane / 32));
+                    f[h2][ks] = Tr::load(a + crow * stride + ks * Tr::KSTEP + Tr::PER_LANE * (lane / 32));
             }
         };
+        if constexpr (!LATE) {
+            coefficients(fa, ad, ad_stride);
+            coefficients(fm, am, am_stride);
+        }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
         const float* grow = gw + 4 * (lane / 32);  // row 8*(r/4) + (r&3) of this lane's half
@@ -203,17 +221,25 @@ __global__ void __launch_bounds__(256, BF16 ? 3 : 1) k_element_mfma(int64_t nc, 
         for (int tile = 0; tile < TPG; ++tile) {
             const int col = (group * TPG + tile) * 32 + (lane & 31);
             floatx16 tot0 = {}, tot1 = {};
-            coefficients(ad, ad_stride);
+            if constexpr (LATE) coefficients(fa, ad, ad_stride);
 #pragma unroll 1
             for (int s = 0; s < MF_NS; ++s) {  // one pair of accumulator chains live at a time
                 floatx16 acc0 = {}, acc1 = {};
                 const E* bs = bl + ((s * TPG + tile) * KS) * WAVE * Tr::PER_LANE + lane * Tr::PER_LANE;
-                if (s == MF_NS - 1) coefficients(am, am_stride);
+                const bool mass = s == MF_NS - 1;
+                if constexpr (LATE) {
+                    if (mass) coefficients(fa, am, am_stride);
+                }
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
                     const F b = Tr::load(bs + ks * WAVE * Tr::PER_LANE);
-                    acc0 = Tr::mma(fa[0][ks], b, acc0);
-                    acc1 = Tr::mma(fa[1][ks], b, acc1);
+                    if constexpr (LATE) {
+                        acc0 = Tr::mma(fa[0][ks], b, acc0);
+                        acc1 = Tr::mma(fa[1][ks], b, acc1);
+                    } else {
+                        acc0 = Tr::mma(mass ? fm[0][ks] : fa[0][ks], b, acc0);
+                        acc1 = Tr::mma(mass ? fm[1][ks] : fa[1][ks], b, acc1);
+                    }
                 }
                 const float4* g0 = reinterpret_cast<const float4*>(grow + s * 32);
                 const float4* g1 = reinterpret_cast<const float4*>(grow + 8 * 32 + s * 32);
@@ -256,11 +282,21 @@ static int launch_mfma(int64_t nc, int ldof, const double* node, const int32_t* 
         set_error("fa_element_matrices_mfma: LDS slice of %zu bytes exceeds 64 KiB", lds);
         return FA_ECAPACITY;
     }
-    const int64_t blocks = ((nc + MF_CELLS_PER_BLOCK - 1) / MF_CELLS_PER_BLOCK + 7) / 8 * 8 * ngroups;
+    const int64_t ranges = (nc + MF_CELLS_PER_BLOCK - 1) / MF_CELLS_PER_BLOCK;
+    const bool deal = ranges >= MF_DEAL_RANGES;
+    const int64_t blocks = (deal ? (ranges + 7) / 8 * 8 : ranges) * ngroups;
     FA_REQUIRE(blocks <= (1 << 24), "fa_element_matrices_mfma: %lld cells are too many", (long long)nc);
-    hipLaunchKernelGGL((k_element_mfma<KS, BF16, TPG>), dim3((unsigned)blocks), dim3(256), lds, s, nc, ldof, node, cell,
-                       static_cast<const E*>(ad), ad_stride, static_cast<const E*>(am), am_stride,
-                       static_cast<const E*>(btab), metric, ld, ngroups, elem);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), lds, s, nc, ldof, node, cell,
+                           static_cast<const E*>(ad), ad_stride, static_cast<const E*>(am), am_stride,
+                           static_cast<const E*>(btab), metric, ld, ngroups, deal, elem);
+    };
+    if constexpr (BF16)
+        launch(k_element_mfma<KS, BF16, TPG, TPG == 1>);
+    else if (ranges * ngroups >= MF_EARLY_FROM && ranges * ngroups < MF_EARLY_TO)
+        launch(k_element_mfma<KS, BF16, TPG, false>);
+    else
+        launch(k_element_mfma<KS, BF16, TPG, true>);
     FA_LAUNCH("k_element_mfma");
     return FA_OK;
 }

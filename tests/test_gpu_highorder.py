@@ -46,3 +46,19 @@ def test_mfma_assembled_matrix_and_cell_coefficient():
     assert torch.equal(A64.col, A32.col) and A32.values.dtype == torch.float32
     err = float((A32.values.double() - A64.values).abs().max()) / float(A64.values.abs().max())
     assert err < 2e-6, err
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (13, 14, 14), (14, 14, 14), (19, 20, 21)])
+@pytest.mark.parametrize("p,q", [(2, 2), (2, 4), (3, 5), (4, 6)])
+@pytest.mark.parametrize("precision,tol", [("fp32", 2e-6), ("bf16", 2e-2)])
+def test_mfma_block_orders(dims, p, q, precision, tol):
+    """6 to 47,880 cells: 1, 30, 33 and 94 ranges of 512 cells (dealt to the XCDs from 32), 1 to 3,666 blocks, slices of
+    one to four tiles; the same bars as above, against the FP64 matrices of the same cells."""
+    mesh = fa.TetrahedronMesh.from_box([0, 1, 0, 1, 0, 1], nx=dims[0], ny=dims[1], nz=dims[2], device=DEV)
+    space = fa.LagrangeFESpace(mesh, p)
+    ref = GroupIntegrator(fa.ScalarDiffusionIntegrator(kx, q=q), fa.ScalarMassIntegrator(1.0, q=q)).assembly(space)
+    m = f"mfma_{precision}"
+    got = GroupIntegrator(fa.ScalarDiffusionIntegrator(kx, q=q, method=m),
+                          fa.ScalarMassIntegrator(1.0, q=q, method=m)).assembly(space, dtype=torch.float32)
+    err = float((got.double() - ref).abs().max()) / float(ref.abs().max())
+    assert err < tol, err
