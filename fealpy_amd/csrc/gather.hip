@@ -15,8 +15,9 @@ __device__ inline int lower_bound_lds(const int32_t* a, int n, int32_t v) {
     return lo;
 }
 
-// G lanes per global row (G >= ldof); each row's columns and accumulators
-// live in LDS.  The incident cells of a row are visited in ascending order
+// G lanes per global row (G >= ldof); each row's columns and FP64 accumulators
+// live in LDS (the sums of k_sum_rows, bit for bit: a pattern's first assembly
+// takes this kernel, the next ones that).  The incident cells of a row are visited in ascending order
 // and lane j adds element entry (i, j) of the current cell, so every CSR entry
 // is summed in ascending cell order -- the order of the reference's stable
 // lexsort + sequential np.add.at.  Distinct columns of one cell never collide.
@@ -30,13 +31,13 @@ __global__ void k_gather_matrix(int64_t gdof, int ldof, const int32_t* __restric
     const int sub = threadIdx.x / G;
     const int lane = threadIdx.x % G;
     int32_t* cols = reinterpret_cast<int32_t*>(smem) + sub * lmax;
-    T* acc = reinterpret_cast<T*>(smem + align_up(sizeof(int32_t) * rpb * lmax, 16)) + sub * lmax;
+    double* acc = reinterpret_cast<double*>(smem + align_up(sizeof(int32_t) * rpb * lmax, 16)) + sub * lmax;
     for (int64_t r = (int64_t)blockIdx.x * rpb + sub; r < gdof; r += (int64_t)gridDim.x * rpb) {
         const int32_t r0 = indptr[r];
         const int L = indptr[r + 1] - r0;
         for (int t = lane; t < L; t += G) {
             cols[t] = indices[r0 + t];
-            acc[t] = T(0);
+            acc[t] = 0.0;
         }
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
@@ -88,7 +89,7 @@ __global__ void k_gather_matrix(int64_t gdof, int ldof, const int32_t* __restric
                 __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
             }
         }
-        for (int t = lane; t < L; t += G) values[r0 + t] = acc[t];
+        for (int t = lane; t < L; t += G) values[r0 + t] = static_cast<T>(acc[t]);
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
     }
@@ -259,16 +260,20 @@ template <class T, int G>
 static int launch_gather(int64_t gdof, int ldof, const int32_t* c2d, const int32_t* ptr, const int32_t* adj,
                          const int32_t* indptr, const int32_t* indices, int lmax, const void* elem, int64_t cstride,
                          void* values, hipStream_t s) {
-    const size_t per_row = sizeof(int32_t) * lmax + sizeof(T) * lmax;
+    const size_t per_row = (sizeof(int32_t) + sizeof(double)) * lmax;
     int rpb = 256 / G;
     while (rpb > 1 && rpb * per_row + 16 > 48 * 1024) rpb >>= 1;
-    const size_t lds = align_up(sizeof(int32_t) * rpb * lmax, 16) + sizeof(T) * rpb * lmax;
-    if (lds > 64 * 1024) {
+    const size_t lds = align_up(sizeof(int32_t) * rpb * lmax, 16) + sizeof(double) * rpb * lmax;
+    if (lds > 160 * 1024) {
         set_error("fa_gather_matrix: row length %d exceeds the LDS capacity", lmax);
         return FA_ECAPACITY;
     }
+    auto k = k_gather_matrix<T, G>;
+    if (lds > 64 * 1024)
+        FA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   static_cast<int>(lds)));
     const unsigned grid = grid_for(gdof, rpb, 1 << 20);
-    hipLaunchKernelGGL((k_gather_matrix<T, G>), dim3(grid), dim3(rpb * G), lds, s, gdof, ldof, c2d, ptr, adj, indptr,
+    hipLaunchKernelGGL(k, dim3(grid), dim3(rpb * G), lds, s, gdof, ldof, c2d, ptr, adj, indptr,
                        indices, lmax, static_cast<const T*>(elem), cstride, static_cast<T*>(values));
     FA_LAUNCH("k_gather_matrix");
     return FA_OK;

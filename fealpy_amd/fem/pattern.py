@@ -29,13 +29,14 @@ def _box_counts(nx, ny, nz):
 
 class Pattern:
     __slots__ = ("cell2dof", "gdof", "ldof", "nc", "_adj_ptr", "_adj", "_max_degree", "indptr", "indices", "nnz",
-                 "max_row", "_maps", "_maps_lock", "_adj_lock", "_pos", "_vpos", "_kept")
+                 "max_row", "_maps", "_maps_lock", "_adj_lock", "_pos", "_vpos", "_kept", "_summed")
 
     def __init__(self, cell2dof, gdof, box=None, kept=False):
         """kept: the pattern of a space, assembled again and again, which
-        keeps the row positions of its incidences (``row_positions``).  box: (nx, ny, nz) of a TetrahedronMesh.from_box P1 map, whose CSR
-        pattern comes from the grid (fa_p1_box_pattern); the incidence lists
-        are then built on first use."""
+        keeps the row positions of its incidences (``row_positions``).  box:
+        (nx, ny, nz) of a TetrahedronMesh.from_box P1 map, whose CSR pattern
+        comes from the grid (fa_p1_box_pattern); the incidence lists are then
+        built on first use."""
         L = nat.lib()
         c2d = cell2dof.to(torch.int32).contiguous()
         nc, ldof = c2d.shape
@@ -47,6 +48,7 @@ class Pattern:
         self._maps_lock = threading.Lock()
         self._pos = self._vpos = None
         self._kept = bool(kept)
+        self._summed = False                              # element matrices have been summed on it once
         if box is not None:
             nx, ny, nz = box
             self.nnz, self.max_row = _box_counts(nx, ny, nz)
@@ -141,10 +143,12 @@ class Pattern:
         ldof^2 a cell: built once and completed on the building stream before
         they are shared.  None for a pattern that is not kept (a region's,
         summed once: it searches the columns as it sums) or has rows over
-        8192 entries."""
+        8192 entries, and while the stream is capturing, which cannot wait."""
         if not self._kept or longest > 8192 or self.nnz == 0 or self.nc == 0:
             return None
         if getattr(self, slot) is None:
+            if torch.cuda.is_current_stream_capturing():
+                return None
             with self._maps_lock:
                 if getattr(self, slot) is None:
                     pos = torch.empty(self.nc * ldof ** 2, dtype=torch.int16, device=self.indptr.device)
@@ -186,7 +190,12 @@ class Pattern:
             elem = elem.contiguous()                      # cells may be padded apart; rows must be dense
         if values is None:
             values = torch.empty(self.nnz, dtype=elem.dtype, device=elem.device)
-        pos = self.row_positions()
+        # the first sum searches the columns: a space assembled once would pay for
+        # the positions (a kernel that searches as long, a wait, 2 ldof^2 bytes a
+        # cell) and not use them.  First call, P2
+        # triangles: 16^2 323 -> 275 us, 192^2 355 -> 284; P3 48^3 3.4 -> 2.6 ms
+        pos = self.row_positions() if self._summed else None
+        self._summed = True
         if pos is not None:
             nat.check(L.fa_sum_rows(nat.dtype_code(elem.dtype), self.gdof, self.ldof, nat.ptr(self.adj_ptr),
                                     nat.ptr(self.adj), nat.ptr(self.indptr), nat.ptr(pos), self.max_row, nat.ptr(elem),

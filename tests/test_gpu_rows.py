@@ -12,6 +12,7 @@ import torch
 
 import fealpy_amd as fa
 from fealpy_amd.fem import integrators, rows
+from fealpy_amd.fem.pattern import pattern_of
 
 pytestmark = pytest.mark.gpu
 DEV = torch.device("cuda")
@@ -131,7 +132,8 @@ def test_long_rows_sum_from_elements(p, n):
     space = fa.LagrangeFESpace(fa.TriangleMesh(fan.node.roll(-1, 0).contiguous(), cell.to(torch.int32)), p)
     it = fa.ScalarDiffusionIntegrator(2.0, q=p + 1)
     for dtype in (torch.float64, torch.float32):
-        _check(fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype), space, it.assembly(space), dtype)
+        for _ in range(2):
+            _check(fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype), space, it.assembly(space), dtype)
 
 
 @pytest.mark.parametrize("name,p,vector", [("tri", 3, False), ("tet", 2, False), ("tri", 4, True), ("tet2", 3, True),
@@ -148,8 +150,32 @@ def test_rows_sum_in_cell_order(name, p, vector, monkeypatch):
         it = fa.LinearElasticityIntegrator(fa.LinearElasticMaterial("m", lame_lambda=1.3, shear_modulus=0.7,
                                                                     **({} if gd == 3 else {"hypo": "plane_strain"})))
         monkeypatch.setattr(rows, "elasticity_values", lambda *a: None)
-    A = fa.BilinearForm(space).add_integrator(it).assembly()
     n, c2d = space.number_of_global_dofs(), space.cell_to_dof().cpu().numpy()
     ref = np.zeros((n, n))
     np.add.at(ref, (c2d[:, :, None], c2d[:, None, :]), it.assembly(space).cpu().numpy())
-    assert np.array_equal(A.to_dense().cpu().numpy(), ref)
+    for _ in range(2):           # the columns searched, then their kept positions
+        assert np.array_equal(fa.BilinearForm(space).add_integrator(it).assembly().to_dense().cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_positions_from_the_second_sum(dtype):
+    """A space assembled once keeps no row positions and waits for nothing; the next sums have the same bits.  While a
+    stream captures nothing is built either."""
+    mesh = MESHES["tet"]()
+    it = fa.ScalarDiffusionIntegrator(2.0, q=3)
+    space = fa.LagrangeFESpace(mesh, 2)
+    first = fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype).values
+    assert pattern_of(space)._pos is None
+    graph, out = torch.cuda.CUDAGraph(), None
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype).values
+    assert pattern_of(space)._pos is None
+    second = fa.BilinearForm(space).add_integrator(it).assembly(dtype=dtype).values
+    assert pattern_of(space)._pos is not None
+    assert torch.equal(first, second)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, first)
