@@ -8,6 +8,7 @@ import torch
 
 from .. import _native as nat
 from .integrators import Integrator
+from .rows import elasticity_tables
 
 _S = slice(None)
 
@@ -16,19 +17,6 @@ def _check_tensor_space(space, who):
     if not hasattr(space, 'scalar_space') or space.dof_ndim != 1 or space.dof_numel != space.GD:
         raise RuntimeError(f"{who} needs a TensorFunctionSpace with shape (-1, GD) or (GD, -1) over a "
                            f"Lagrange space")
-
-
-def _precontracted(space, q):
-    """M[i, j, m, n] = sum_q w_q R[q, i, m] R[q, j, n] (FP64, on the device),
-    cached per quadrature index, complete before another stream or thread can see it."""
-    ss = space.scalar_space
-    cache = ss.__dict__.setdefault('_elast_M', {})
-    if q not in cache:
-        _, qw, _, R = ss.tables(q)                                   # R: (NQ, ldof, TD+1)
-        M = torch.einsum('q, qim, qjn -> ijmn', qw, R, R).contiguous()
-        torch.cuda.current_stream(M.device).synchronize()
-        cache[q] = M
-    return cache[q]
 
 
 class LinearElasticityIntegrator(Integrator):
@@ -63,7 +51,7 @@ class LinearElasticityIntegrator(Integrator):
         mesh = ss.mesh
         sel = self.entity_selection(indices)
         q = ss.p + 3 if self.q is None else self.q
-        M = _precontracted(space, q)
+        M = elasticity_tables(ss, q)[0]
         cell = mesh.cell[sel].to(torch.int32).contiguous()
         nc = cell.shape[0]
         ldof = ss.number_of_local_dofs()

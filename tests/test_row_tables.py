@@ -1,8 +1,8 @@
-"""Reference tables of the row kernels (rows.p1_table, rows.elasticity_table):
-formed on the host and complete when they are published, each entry within half
-a unit in the last place of the exact sum of the rule's numbers (the sums have
-64 bits of mantissa, which adds less than a tenth of a unit; a P1 entry adds two
-of them)."""
+"""Reference tables of the row kernels: p1_table formed on the host and complete
+when it is published, each entry the exact sum of the rule's numbers to half a
+unit in the last place (and a tenth, for sums of 64 mantissa bits); the
+elasticity table the element kernel's, reduced, within (NQ + 4) units of that
+table's largest entry."""
 from fractions import Fraction
 
 import numpy as np
@@ -28,24 +28,26 @@ def _exact(space, q):
     return np.einsum("q,qia,qjb->abij", w, R, R), np.einsum("q,qi,qj->ij", w, phi, phi)
 
 
-def _within(got, exact, ulps):
-    for g, e in zip(got.reshape(-1).tolist(), exact.reshape(-1)):
-        scale = max(abs(float(e)), 1e-3)       # entries that cancel: relative to the terms, of order 1
-        assert abs(Fraction(g) - e) <= Fraction(ulps * 2.0 ** -52 * scale)
+@pytest.mark.parametrize("td,q", [(2, 2), (2, 4), (3, 2), (3, 4), (3, 6)])
+def test_p1_table_is_exact_to_rounding(td, q):
+    space = _space(td, 1)
+    M, mass = _exact(space, q)
+    pairs = [(a, b) for a in range(td) for b in range(a, td)]
+    exact = np.stack([M[a, b] if a == b else M[a, b] + M[b, a] for a, b in pairs] + [mass])
+    for g, e in zip(rows.p1_table(space, q).reshape(-1).tolist(), exact.reshape(-1)):
+        assert abs(Fraction(g) - e) <= Fraction(1.1 * 2.0 ** -53 * max(abs(float(e)), 1e-3))
 
 
 @pytest.mark.parametrize("td,p,q", [(2, 1, 4), (3, 1, 4), (2, 2, 5), (3, 2, 5), (2, 4, 7)])
-def test_tables_are_exact_to_rounding(td, p, q):
+def test_elasticity_table_reduces_the_element_kernels(td, p, q):
     space = _space(td, p)
-    M, mass = _exact(space, q)
-    _within(rows.elasticity_table(space, q), M, 0.6)
-    if p == 1:
-        pairs = [(a, b) for a in range(td) for b in range(a, td)]
-        exact = np.stack([M[a, b] if a == b else M[a, b] + M[b, a] for a, b in pairs] + [mass])
-        _within(rows.p1_table(space, q), exact, 1.6)
+    M, reduced = rows.elasticity_tables(space, q)
+    nq = len(rows._rule(space, q)[1])
+    exact = np.vectorize(float)(_exact(space, q)[0])
+    assert float(np.abs(reduced.numpy() - exact).max()) <= (nq + 4) * 2.0 ** -52 * float(M.abs().max())
 
 
-def test_tables_queue_no_device_work(monkeypatch):
+def test_p1_table_queues_no_device_work(monkeypatch):
     """A kernel of the building stream would leave the published table incomplete for any other stream."""
     def refuse(*args, **kw):
         raise AssertionError("a table formed by queued tensor operations")
@@ -54,4 +56,3 @@ def test_tables_queue_no_device_work(monkeypatch):
     for name in ("einsum", "stack", "matmul"):
         monkeypatch.setattr(torch, name, refuse)
     rows.p1_table(space, 3)
-    rows.elasticity_table(space, 3)
