@@ -210,6 +210,20 @@ def _fused_scalar_group(ints):
 MFMA_METHODS = {'mfma_bf16': 'bf16', 'mfma_fp32': 'fp32'}
 
 
+# A separable coefficient is sampled by a kernel of its own (fa_sep_sample) where
+# the element kernel, whose registers hold its accumulators, would lose more by
+# evaluating it than the launch costs: from 600,000 points (P2 triangles 0.49M
+# points 69 us sampled against 62 us, 1.2M points 73 against 76; P2 tetrahedra
+# 0.36M 69 against 62, 1.2M 95 against 100) and for elements of 20 functions and
+# more at any size (P3 tetrahedra 73,000 points 107 against 113 us, 1.4M 184
+# against 220; P4 199 against 207, 618 against 650).  The values are the same.
+SEP_SAMPLE_MIN_POINTS = 600_000
+
+
+def _sampled_first(points, ldof):
+    return points >= SEP_SAMPLE_MIN_POINTS or ldof >= 20
+
+
 def _scalar_elements(space, ops, *, indices=None, selection=_S, dtype=None):
     L = nat.lib()
     mesh = space.mesh
@@ -233,7 +247,7 @@ def _scalar_elements(space, ops, *, indices=None, selection=_S, dtype=None):
     for op, it in ops:
         spec[op] = coef_spec(it.coef, space, q, selection, allow_sep=True)
     for op, (kind, scale, table) in spec.items():
-        if kind == nat.COEF_SEP:     # sampled first: the element kernel's registers hold its accumulators
+        if kind == nat.COEF_SEP and _sampled_first(nc * qw.shape[0], ldof):
             vals = torch.empty((nc, qw.shape[0]), dtype=torch.float64, device=space.device)
             nat.check(L.fa_sep_sample(space.TD, qw.shape[0], nat.ptr(mesh.node), nat.ptr(cell), nc, nat.ptr(table),
                                       nat.ptr(vals), nat.stream()), "fa_sep_sample")

@@ -11,6 +11,7 @@ import torch
 
 import fealpy_amd as fa
 from fealpy_amd import expr
+from fealpy_amd.fem import integrators
 from fealpy_amd.functionspace.basis import grad_shape_function, shape_function
 
 pytestmark = pytest.mark.gpu
@@ -117,3 +118,16 @@ def test_reference_sums_keep_their_precision(td, p, q, op):
     cls = fa.ScalarDiffusionIntegrator if op == "diff" else fa.ScalarMassIntegrator
     got = cls(torch.ones(1, dtype=torch.float64, device=DEV), q=q).assembly(fa.LagrangeFESpace(mesh, p))[0].cpu().numpy()
     assert np.sqrt(((got - ref) ** 2).sum() / (ref ** 2).sum()) <= 2 * 2.0 ** -53
+
+
+@pytest.mark.parametrize("dims,p", [((5, 4), 2), ((2, 3, 2), 2), ((1, 2, 1), 3), ((3, 3), 4)])
+def test_separable_coefficient_sampled_or_in_the_kernel(dims, p, monkeypatch):
+    """Both routes evaluate the same factors in the same order: the same bits."""
+    space = fa.LagrangeFESpace(_mesh(dims), p)
+    f = 1.0 + 0.5 * expr.sin(math.pi * expr.x) * expr.cos(2.0 * expr.y) + expr.exp(expr.x) * expr.y
+    it = fa.ScalarDiffusionIntegrator(f, q=p + 2)
+    out = []
+    for sampled in (True, False):
+        monkeypatch.setattr(integrators, "_sampled_first", lambda points, ldof: sampled)
+        out.append(it.assembly(space))
+    assert torch.equal(out[0], out[1])

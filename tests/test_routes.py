@@ -13,3 +13,10 @@ ONE = 2.0 * expr.sin(expr.x) * expr.cos(expr.y) * expr.exp(expr.z)
 def test_one_pass_load_vector_of_a_box(source, nq, n, one_pass):
     """Only one-term sources at the four-point rule on large grids: the others lost up to six times."""
     assert integrators._box_one_pass(source, nq, 6 * n ** 3) is one_pass
+
+
+@pytest.mark.parametrize("points,ldof,sampled", [(7_680, 6, False), (490_000, 10, False), (1_200_000, 6, True),
+                                                 (45_000, 20, True), (100_000, 35, True)])
+def test_separable_coefficient_sampled_first(points, ldof, sampled):
+    """A launch more only where it gains: small P2 assemblies lost a tenth by it."""
+    assert integrators._sampled_first(points, ldof) is sampled
