@@ -133,37 +133,6 @@ __device__ inline T group_sum(T v) {
     return v;
 }
 
-// Sum of a row's products of type T, given in FP64.  FP32's fit it exactly and
-// are added plainly; FP64's keep what the additions round off (Knuth's two-sum),
-// so that s + c is the sum of the terms to a rounding, however many they are and
-// in whichever order.
-template <class T>
-struct RowSum {
-    static constexpr bool COMP = sizeof(T) == 8;
-    double s = 0.0, c = 0.0;
-    __device__ void add(double v) {
-        const double t = s + v;
-        if constexpr (COMP) {
-            const double b = t - s;
-            c += (s - (t - b)) + (v - b);
-        }
-        s = t;
-    }
-    // over an aligned group of G lanes (G power of two <= 64); all hold the result
-    template <int G>
-    __device__ double group() {
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1) {
-            const double other = COMP ? __shfl_xor(c, o) : 0.0;
-            add(__shfl_xor(s, o));
-            if constexpr (COMP) c += other;
-        }
-        if constexpr (!COMP) return s;
-        const double r = s + c;
-        return r == r ? r : s;  // infinite terms: their plain sum (c is NaN)
-    }
-};
-
 // inclusive scan inside an aligned group of G lanes
 template <int G>
 __device__ inline int group_inclusive_scan(int v) {
