@@ -133,6 +133,49 @@ __device__ inline T group_sum(T v) {
     return v;
 }
 
+// the value of lane ^ o; within a quad by a register move, no LDS instruction.
+// The lanes of a group are all active.
+template <int CTRL>
+__device__ inline double quad_perm(double v) {
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+    return __hiloint2double(hi, lo);
+}
+__device__ inline double lane_xor(double v, int o) {
+    return o == 1 ? quad_perm<0xB1>(v) : o == 2 ? quad_perm<0x4E>(v) : __shfl_xor(v, o);
+}
+
+// Sum of a row's products of type T, given in FP64.  FP32's fit it exactly and
+// are added plainly; FP64's keep what the additions round off (Knuth's two-sum),
+// so that s + c is the sum of the terms to a rounding, however many they are and
+// in whichever order.
+template <class T>
+struct RowSum {
+    static constexpr bool COMP = sizeof(T) == 8;
+    double s = 0.0, c = 0.0;
+    __device__ void add(double v) {
+        const double t = s + v;
+        if constexpr (COMP) {
+            const double b = t - s;
+            c += (s - (t - b)) + (v - b);
+        }
+        s = t;
+    }
+    // over an aligned group of G lanes (G power of two <= 64); all hold the result
+    template <int G>
+    __device__ double group() {
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) {
+            const double other = COMP ? lane_xor(c, o) : 0.0;
+            add(lane_xor(s, o));
+            if constexpr (COMP) c += other;
+        }
+        if constexpr (!COMP) return s;
+        const double r = s + c;
+        return r == r ? r : s;  // infinite terms: their plain sum (c is NaN)
+    }
+};
+
 // inclusive scan inside an aligned group of G lanes
 template <int G>
 __device__ inline int group_inclusive_scan(int v) {

@@ -11,7 +11,12 @@ namespace fa {
 // A block takes 256 / G consecutive rows, whose entries are one contiguous
 // range: it reads that range whole lines at a time whatever the rows' lengths,
 // four entries a thread in flight, leaves the products in LDS, and G lanes a
-// row add the row's.  What bounds it is HBM: 12 (8 in FP32) bytes an entry.
+// row add the row's.  What bounds it is HBM: 12 (8 in FP32) bytes an entry, so
+// the sums can afford to lose nothing: FP32 products are kept exact in FP64, and
+// the additions keep what they round off (RowSum).  An FP64 product is rounded
+// once, where lanes that read a row themselves rounded every partial sum.  Off 64
+// bits, 40^3 P2 tetrahedra: FP64 3.9e-16 with 32 lanes a row, 4.8e-16 with 4 that
+// add plainly, 3.8e-16 so; FP32 8.0e-8, 7.2e-8, 4.1e-8.
 // The form with G lanes reading each row themselves lost them in the rows'
 // remainders and waited for one entry at a time: a P2 tetrahedral matrix
 // (885k rows of 18 to 65 entries, FP64) 141 -> 73 us, 4.4 TB/s.
@@ -22,13 +27,13 @@ __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t* __restri
                                              const int32_t* __restrict__ indices, const T* __restrict__ vals,
                                              const T* __restrict__ x, T* __restrict__ y) {
     constexpr int RB = 256 / G;
-    __shared__ T prod[STREAM];
+    __shared__ double prod[STREAM];
     const int lane = threadIdx.x % G;
     for (int64_t r0 = (int64_t)xcd_window_block() * RB; r0 < n; r0 += (int64_t)gridDim.x * RB) {
         const int64_t end = min(r0 + RB, n), r = min(r0 + threadIdx.x / G, end);
         const int32_t e0 = indptr[r0], e1 = indptr[end];
         const int32_t k0 = indptr[r], k1 = indptr[min(r + 1, end)];
-        T s = T(0);
+        RowSum<T> s;
         for (int32_t e = e0; e < e1; e += STREAM) {
             const int m = min(STREAM, e1 - e);
             for (int b = 0; b < m; b += 1024) {
@@ -45,14 +50,14 @@ __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t* __restri
                 for (int u = 0; u < 4; ++u) w[u] = x[c[u]];
 #pragma unroll
                 for (int u = 0; u < 4; ++u)
-                    if (b + u * 256 + (int)threadIdx.x < m) prod[b + u * 256 + threadIdx.x] = v[u] * w[u];
+                    if (b + u * 256 + (int)threadIdx.x < m) prod[b + u * 256 + threadIdx.x] = static_cast<double>(v[u]) * w[u];
             }
             __syncthreads();
-            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s += prod[k - e];
+            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s.add(prod[k - e]);
             __syncthreads();
         }
-        s = group_sum<G>(s);
-        if (lane == 0 && r < end) y[r] = s;
+        const double t = s.template group<G>();
+        if (lane == 0 && r < end) y[r] = static_cast<T>(t);
     }
 }
 
@@ -137,14 +142,14 @@ __global__ void __launch_bounds__(256) k_bc_count(int64_t n, const int32_t* __re
 // order); VAL 2: the values on A's own pattern (boundary rows 1 on the diagonal
 // and 0 elsewhere, boundary columns 0; nval may be vals itself: a chunk is read
 // before any of it is written); VAL 0: none.  RHS: out = f - A uh, uh on
-// boundary rows, summed in one order whatever VAL.  As in k_spmv a block streams the contiguous entries of 256 / G rows;
-// the kept ones' new places are contiguous too: the first row's, plus the kept
-// entries before (ballots, a prefix over the block's waves), so values leave
-// in order.  Of a boundary row the first entry keeps a place, for the row's
-// thread to fill; a boundary row without entries has none, and the block that
-// sees its count fall short places its rows one by one.  nidx == NULL refills
-// values only; U: the type of the filtered values (an FP32 copy of an FP64
-// matrix is rounded once).  Both directions of HBM bound it: 20 bytes an entry.
+// boundary rows, summed in one order whatever VAL and as precisely as k_spmv's.
+// As there a block streams the contiguous entries of 256 / G rows; the kept ones'
+// new places are contiguous too: the first row's, plus the kept entries before
+// (ballots, a prefix over the block's waves), so values leave in order.  Of a
+// boundary row the first entry keeps a place, for the row's thread to fill; a
+// boundary row without entries has none, and the block that sees its count fall
+// short places its rows one by one.  nidx == NULL refills values only; U: the
+// type of the filtered values (an FP32 copy of an FP64 matrix is rounded once).  Both directions of HBM bound it: 20 bytes an entry.
 // 15.0M entries (100 x 113 x 90 cells, P1): 16 lanes a row 128 -> 75 us.
 template <class T, class U, int G, int VAL, bool RHS>
 __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __restrict__ indptr,
@@ -154,7 +159,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
                                                 const T* __restrict__ uh, const T* __restrict__ f,
                                                 T* __restrict__ out) {
     constexpr int RB = 256 / G, CH = STREAM / 2, PER = CH / 256, WAVES = 256 / WAVE;
-    __shared__ T prod[RHS ? CH : 1];
+    __shared__ double prod[RHS ? CH : 1];
     __shared__ uint8_t mark[CH];  // 1: entry of a boundary row, 2: its first
     __shared__ int cnt[PER * WAVES];
     const int lane = threadIdx.x % G, wave = threadIdx.x / WAVE;
@@ -166,7 +171,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
         const int32_t o0 = VAL == 1 ? nptr[r0] : 0, o1 = VAL == 1 ? nptr[end] : 0;
         const bool fixed = r < end && bd[r] != 0;
         int32_t at = o0;
-        T s = T(0);
+        RowSum<T> s;
         for (int32_t e = e0; e < e1; e += CH) {
             const int m = min(CH, e1 - e);
             reinterpret_cast<uint32_t*>(mark)[threadIdx.x] = 0;
@@ -210,7 +215,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
                     if (mk == 0) nval[e + i] = cb[u] ? U(0) : static_cast<U>(v[u]);
                 }
                 if constexpr (RHS) {
-                    if (i < m) prod[i] = v[u] * w[u];
+                    if (i < m) prod[i] = static_cast<double>(v[u]) * w[u];
                 }
             }
             __syncthreads();
@@ -227,7 +232,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
                     }
             }
             if constexpr (RHS)
-                for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s += prod[k - e];
+                for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s.add(prod[k - e]);
             __syncthreads();
         }
         if (at != o1) {  // a boundary row without entries, the same for the whole block
@@ -241,14 +246,15 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
             }
             __syncthreads();
         }
-        if constexpr (RHS) s = group_sum<G>(s);
+        double Auh = 0.0;
+        if constexpr (RHS) Auh = s.template group<G>();
         if (lane == 0 && r < end) {
             if (VAL == 1 && fixed) {
                 const int32_t o = nptr[r];
                 if (nidx) nidx[o] = static_cast<int32_t>(r);
                 nval[o] = U(1);
             }
-            if constexpr (RHS) out[r] = fixed ? uh[r] : f[r] - s;
+            if constexpr (RHS) out[r] = fixed ? uh[r] : static_cast<T>(f[r] - Auh);
         }
     }
 }
@@ -496,7 +502,7 @@ __global__ void __launch_bounds__(256) k_csr_residual(int64_t n, const int32_t* 
         const int64_t rr = min(r, n - 1);
         const double bv = b[rr];
         const bool fixed = bd[rr] != 0;
-        double s = 0.0;
+        RowSum<double> s;
         for (int32_t e = e0; e < e1; e += STREAM) {
             const int m = min(STREAM, e1 - e);
             for (int q = 0; q < m; q += 1024) {
@@ -515,11 +521,11 @@ __global__ void __launch_bounds__(256) k_csr_residual(int64_t n, const int32_t* 
                     if (q + u * 256 + (int)threadIdx.x < m) prod[q + u * 256 + threadIdx.x] = v[u] * w[u];
             }
             __syncthreads();
-            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s += prod[k - e];
+            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s.add(prod[k - e]);
             __syncthreads();
         }
-        s = group_sum<G>(s);
-        const double t = fixed ? 0.0 : bv - s;
+        const double Ax = s.template group<G>();
+        const double t = fixed ? 0.0 : bv - Ax;
         if (lane == 0 && r < end) {
             y[r] = static_cast<Y>(t);
             nrm += t * t;

@@ -84,3 +84,40 @@ def test_dirichlet_forms(n, mean, long_row):
     ref = np.where(bd, uh, f - S @ uh)
     bound = 2.2e-16 * (np.diff(crow) + 3) * (abs(S) @ np.abs(uh) + np.abs(f) + np.abs(uh))
     assert np.all(np.abs(out.cpu().numpy() - ref) <= bound)
+
+
+@pytest.mark.parametrize("mean,long_row", [(7, 0), (40, 0), (9, 5000)])
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_row_sums_lose_nothing(mean, long_row, dtype):
+    """FP32 products and sums are exact but for the result's rounding; FP64 ones but for each product's and the result's,
+    whatever the row's length (positive terms, so that their size is the result's)."""
+    n = 6000
+    crow, col, val = _matrix(n, mean, n + mean, long_row)
+    v, x = (torch.as_tensor(np.abs(a), dtype=dtype) for a in (val, np.random.default_rng(1).standard_normal(n)))
+    ptr = [torch.as_tensor(a, device=DEV) for a in (crow, col)]
+    A = fa.CSRTensor(*ptr, v.to(DEV), (n, n))
+    terms = v.numpy().astype(np.longdouble) * x.numpy()[col].astype(np.longdouble)
+    ref = np.zeros(n, np.longdouble)
+    np.add.at(ref, np.repeat(np.arange(n), np.diff(crow)), terms)
+    half = 2.0 ** -53 if dtype == torch.float64 else 2.0 ** -24
+    bound = half * (2.01 if dtype == torch.float64 else 1.01) * ref
+    assert np.all(np.abs((A @ x.to(DEV)).cpu().numpy().astype(np.longdouble) - ref) <= bound)
+    if dtype == torch.float64:                    # the right-hand side's A uh: one rounding more, of f - A uh
+        out = torch.empty(n, dtype=dtype, device=DEV)
+        zero, bd = torch.zeros(n, dtype=dtype, device=DEV), torch.zeros(n, dtype=torch.uint8, device=DEV)
+        p, xd, vd = nat.ptr, x.to(DEV), v.to(DEV)
+        nat.check(nat.lib().fa_dirichlet_rhs(0, n, p(ptr[0]), p(ptr[1]), p(vd), p(bd), p(xd), p(zero), p(out),
+                                             nat.stream()))
+        assert np.all(np.abs(out.cpu().numpy().astype(np.longdouble) + ref) <= bound)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("terms,expected", [([np.inf, 1.0, 2.0], np.inf), ([1.0, -np.inf, 3.0], -np.inf),
+                                            ([np.inf, -np.inf, 1.0], np.nan), ([1.0, np.nan, 2.0], np.nan)])
+def test_infinite_terms(terms, expected, dtype):
+    """Row 1 of three holds the terms; its neighbours stay as they are."""
+    crow = torch.tensor([0, 1, 4, 5], dtype=torch.int32, device=DEV)
+    col = torch.tensor([0, 0, 1, 2, 2], dtype=torch.int32, device=DEV)
+    val = torch.tensor([2.0, *terms, 3.0], dtype=dtype, device=DEV)
+    y = (fa.CSRTensor(crow, col, val, (3, 3)) @ torch.ones(3, dtype=dtype, device=DEV)).cpu().numpy()
+    np.testing.assert_array_equal(y, np.array([2.0, expected, 3.0]))
