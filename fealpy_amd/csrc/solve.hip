@@ -20,7 +20,7 @@ namespace fa {
 // The form with G lanes reading each row themselves lost them in the rows'
 // remainders and waited for one entry at a time: a P2 tetrahedral matrix
 // (885k rows of 18 to 65 entries, FP64) 141 -> 73 us, 4.4 TB/s.
-constexpr int STREAM = 2048;  // products held at once
+constexpr int STREAM = 2048;  // products held at once; no index passes the range's end, which may be near 2^31
 
 template <class T, int G>
 __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t* __restrict__ indptr,
@@ -34,8 +34,7 @@ __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t* __restri
         const int32_t e0 = indptr[r0], e1 = indptr[end];
         const int32_t k0 = indptr[r], k1 = indptr[min(r + 1, end)];
         RowSum<T> s;
-        for (int32_t e = e0; e < e1; e += STREAM) {
-            const int m = min(STREAM, e1 - e);
+        for (int32_t e = e0, m; (m = min(STREAM, e1 - e)) > 0; e += m) {
             for (int b = 0; b < m; b += 1024) {
                 int32_t c[4];
                 T v[4];
@@ -53,7 +52,7 @@ __global__ void __launch_bounds__(256) k_spmv(int64_t n, const int32_t* __restri
                     if (b + u * 256 + (int)threadIdx.x < m) prod[b + u * 256 + threadIdx.x] = static_cast<double>(v[u]) * w[u];
             }
             __syncthreads();
-            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s.add(prod[k - e]);
+            for (int i = max(k0 - e, 0) + lane; i < min(k1 - e, m); i += G) s.add(prod[i]);
             __syncthreads();
         }
         const double t = s.template group<G>();
@@ -160,7 +159,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
                                                 T* __restrict__ out) {
     constexpr int RB = 256 / G, CH = STREAM / 2, PER = CH / 256, WAVES = 256 / WAVE;
     __shared__ double prod[RHS ? CH : 1];
-    __shared__ uint8_t mark[CH];  // 1: entry of a boundary row, 2: its first
+    __shared__ alignas(4) uint8_t mark[CH];  // 1: entry of a boundary row, 2: its first
     __shared__ int cnt[PER * WAVES];
     const int lane = threadIdx.x % G, wave = threadIdx.x / WAVE;
     const unsigned long long below = (1ull << (threadIdx.x % WAVE)) - 1;
@@ -172,8 +171,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
         const bool fixed = r < end && bd[r] != 0;
         int32_t at = o0;
         RowSum<T> s;
-        for (int32_t e = e0; e < e1; e += CH) {
-            const int m = min(CH, e1 - e);
+        for (int32_t e = e0, m; (m = min(CH, e1 - e)) > 0; e += m) {
             reinterpret_cast<uint32_t*>(mark)[threadIdx.x] = 0;
             int32_t c[PER];
             T v[PER], w[PER];
@@ -186,7 +184,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
             }
             __syncthreads();
             if (fixed)
-                for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) mark[k - e] = k == k0 ? 2 : 1;
+                for (int i = max(k0 - e, 0) + lane; i < min(k1 - e, m); i += G) mark[i] = e + i == k0 ? 2 : 1;
 #pragma unroll
             for (int u = 0; u < PER; ++u) {
                 cb[u] = bd[c[u]] != 0;
@@ -195,8 +193,8 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
             __syncthreads();
             if constexpr (VAL == 2) {
                 if (fixed)
-                    for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G)
-                        nval[k] = indices[k] == r ? U(1) : U(0);
+                    for (int i = max(k0 - e, 0) + lane; i < min(k1 - e, m); i += G)
+                        nval[e + i] = indices[e + i] == r ? U(1) : U(0);
             }
             bool keep[PER];
             int rank[PER];
@@ -232,7 +230,7 @@ __global__ void __launch_bounds__(256) k_bc_rows(int64_t n, const int32_t* __res
                     }
             }
             if constexpr (RHS)
-                for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s.add(prod[k - e]);
+                for (int i = max(k0 - e, 0) + lane; i < min(k1 - e, m); i += G) s.add(prod[i]);
             __syncthreads();
         }
         if (at != o1) {  // a boundary row without entries, the same for the whole block
@@ -503,8 +501,7 @@ __global__ void __launch_bounds__(256) k_csr_residual(int64_t n, const int32_t* 
         const double bv = b[rr];
         const bool fixed = bd[rr] != 0;
         RowSum<double> s;
-        for (int32_t e = e0; e < e1; e += STREAM) {
-            const int m = min(STREAM, e1 - e);
+        for (int32_t e = e0, m; (m = min(STREAM, e1 - e)) > 0; e += m) {
             for (int q = 0; q < m; q += 1024) {
                 int32_t c[4];
                 double v[4], w[4];
@@ -521,7 +518,7 @@ __global__ void __launch_bounds__(256) k_csr_residual(int64_t n, const int32_t* 
                     if (q + u * 256 + (int)threadIdx.x < m) prod[q + u * 256 + threadIdx.x] = v[u] * w[u];
             }
             __syncthreads();
-            for (int32_t k = max(k0, e) + lane; k < min(k1, e + m); k += G) s.add(prod[k - e]);
+            for (int i = max(k0 - e, 0) + lane; i < min(k1 - e, m); i += G) s.add(prod[i]);
             __syncthreads();
         }
         const double Ax = s.template group<G>();
