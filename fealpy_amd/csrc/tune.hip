@@ -37,7 +37,9 @@ extern "C" int fa_tune_key(int family, int64_t a, int64_t b) {
     switch (family) {
         case FA_TUNE_SPMV_LANES: {  // a = rows, b = entries: average row length class
             const double avg = a > 0 ? double(b) / double(a) : 1.0;
-            return avg <= 6 ? 0 : avg <= 12 ? 1 : avg <= 24 ? 2 : avg <= 48 ? 3 : 4;
+            int k = 0;  // one class for each of the kernel's built-in choices (8 entries a row and lane)
+            while (k < 6 && avg > 8.0 * (1 << k)) ++k;
+            return k;
         }
         case FA_TUNE_SUM_ROWS_LANES:  // a = topological dimension, b = longest CSR row
             return static_cast<int>((a == 3 ? 4 : 0) + (b <= 16 ? 0 : b <= 32 ? 1 : b <= 64 ? 2 : 3));

@@ -25,8 +25,8 @@ from . import _native as nat
 SPMV_LANES = 0           # FA_TUNE_SPMV_LANES
 SUM_ROWS_LANES = 1       # FA_TUNE_SUM_ROWS_LANES
 
-CANDIDATES = {SPMV_LANES: (4, 8, 16, 32, 64), SUM_ROWS_LANES: (4, 8, 16, 32)}
-FAMILY_NAMES = {SPMV_LANES: "spmv_sum_lanes", SUM_ROWS_LANES: "sum_rows_lanes"}
+CANDIDATES = {SPMV_LANES: (1, 2, 4, 8, 16, 32, 64), SUM_ROWS_LANES: (4, 8, 16, 32)}
+FAMILY_NAMES = {SPMV_LANES: "spmv_row_lanes", SUM_ROWS_LANES: "sum_rows_lanes"}
 
 _DEFAULT_PATH = os.path.join(os.path.expanduser("~"), ".cache", "fealpy_amd", "tune.json")
 

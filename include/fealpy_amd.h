@@ -853,7 +853,7 @@ int fa_pcg_graph(int dtype, const fa_sell_t* A, const fa_mg_t* M, const void* b,
  * Tile shapes chosen by the project autotuner (fealpy_amd/tune.py), which
  * times the candidates of a kernel family on the caller's own operator and
  * stores the fastest here; no counterpart in the reference.  Families:
- *   FA_TUNE_SPMV_LANES      lanes per CSR row of fa_spmv (4..64), keyed by the
+ *   FA_TUNE_SPMV_LANES      lanes per CSR row of fa_spmv (1..64), keyed by the
  *                           average row length class (fa_tune_key(f, n, nnz));
  *   FA_TUNE_SUM_ROWS_LANES  lanes per CSR row of P1 assembly pass 2
  *                           (fa_sum_incidence_rows: 4, 8, 16 or 32), keyed by

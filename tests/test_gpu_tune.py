@@ -69,6 +69,33 @@ def test_spmv_lanes(tmp_path):
         nat.check(L.fa_tune_set(SPMV_LANES, key, 0), "fa_tune_set")
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("mean", [1, 3, 8, 9, 16, 17, 40, 130, 300])
+def test_spmv_every_lane_count_is_a_candidate(mean, dtype):
+    """The built-in choice is among the candidates, one class each, and every candidate gives the same product."""
+    L, n = nat.lib(), 400
+    key = L.fa_tune_key(SPMV_LANES, n, n * mean)
+    default = next(g for g in (1, 2, 4, 8, 16, 32, 64) if g == 64 or mean <= 8 * g)
+    assert default in CANDIDATES[SPMV_LANES] and key == (1, 2, 4, 8, 16, 32, 64).index(default)
+    g = np.random.default_rng(mean)
+    col = np.stack([np.sort(g.choice(n, mean, replace=False)) for _ in range(n)])
+    val = g.standard_normal((n, mean))
+    A = fa.CSRTensor(torch.arange(n + 1, dtype=torch.int32, device=DEV) * mean,
+                     torch.as_tensor(col.reshape(-1), dtype=torch.int32, device=DEV),
+                     torch.as_tensor(val.reshape(-1), dtype=dtype, device=DEV), (n, n))
+    x = torch.as_tensor(g.standard_normal(n), dtype=dtype, device=DEV)
+    v, xs = A.values.cpu().double().numpy().reshape(n, mean), x.cpu().double().numpy()
+    ref, size = (v * xs[col]).sum(1), (np.abs(v * xs[col])).sum(1)
+    eps = 2.2e-16 if dtype == torch.float64 else 6e-8
+    try:
+        for lanes in (0, *CANDIDATES[SPMV_LANES]):
+            nat.check(L.fa_tune_set(SPMV_LANES, key, lanes), "fa_tune_set")
+            # FP64: the reference adds `mean` terms; FP32: one rounding of the result
+            assert np.all(np.abs((A @ x).cpu().double().numpy() - ref) <= eps * (mean if eps < 1e-9 else 1.01) * size)
+    finally:
+        nat.check(L.fa_tune_set(SPMV_LANES, key, 0), "fa_tune_set")
+
+
 def test_tune_set_rejects_bad_family():
     L = nat.lib()
     assert L.fa_tune_set(7, 0, 8) == nat.FA_EINVAL
