@@ -14,6 +14,7 @@ count, so its results move at the rounding level with the choice (a cached
 choice keeps them identical from run to run).
 """
 import json
+import math
 import os
 import statistics
 import threading
@@ -130,7 +131,8 @@ class Autotuner:
         space's pattern, timing a whole two-pass assembly of a diffusion form
         (also on a from_box mesh, whose own matrices take the structured
         kernel: the choice serves the meshes with this row length that do
-        not).  Not thread-safe: the two-pass route is forced for the duration."""
+        not, and coefficients that vary on a cell).  Not thread-safe: the
+        two-pass route is forced for the duration."""
         from .fem import BilinearForm, ScalarDiffusionIntegrator, integrators
         from .fem.pattern import pattern_of
         L = nat.lib()
@@ -140,12 +142,14 @@ class Autotuner:
 
         def run():
             form.assembly(dtype=dtype)
-        box, two = integrators.BOX_ASSEMBLY, integrators.TWO_PASS_MIN_CELLS
-        integrators.BOX_ASSEMBLY, integrators.TWO_PASS_MIN_CELLS = False, 0
+        names = ("BOX_ASSEMBLY", "TWO_PASS_MIN_CELLS", "RECORDS_MIN_CELLS")
+        old = [getattr(integrators, n) for n in names]
+        integrators.BOX_ASSEMBLY, integrators.TWO_PASS_MIN_CELLS, integrators.RECORDS_MIN_CELLS = False, 0, math.inf
         try:
             return self.tune(SUM_ROWS_LANES, key, run, device=space.device)
         finally:
-            integrators.BOX_ASSEMBLY, integrators.TWO_PASS_MIN_CELLS = box, two
+            for n, v in zip(names, old):
+                setattr(integrators, n, v)
 
 
 _default = None

@@ -48,6 +48,25 @@ def test_assembly_lanes_bitwise_and_cached(tmp_path, monkeypatch):
         nat.check(L.fa_tune_set(SUM_ROWS_LANES, key, 0), "fa_tune_set")
 
 
+def test_assembly_tuning_times_the_two_passes(monkeypatch):
+    """Also on a mesh large enough to be assembled from a record per cell, where the lane count changes nothing."""
+    from fealpy_amd.fem import integrators
+    monkeypatch.setattr(integrators, "RECORDS_MIN_CELLS", 0)
+
+    def refuse(*args):
+        raise AssertionError("rows from records")
+    monkeypatch.setattr(integrators, "p1_values", refuse)
+    space = fa.LagrangeFESpace(fa.TetrahedronMesh.from_box(nx=5, ny=4, nz=3, device=DEV), 1)
+    L = nat.lib()
+    from fealpy_amd.fem.pattern import pattern_of
+    key = L.fa_tune_key(SUM_ROWS_LANES, 3, pattern_of(space).max_row)
+    try:
+        Autotuner(path=None, reps=1).tune_assembly(space, q=2)
+    finally:
+        nat.check(L.fa_tune_set(SUM_ROWS_LANES, key, 0), "fa_tune_set")
+    assert integrators.RECORDS_MIN_CELLS == 0 and integrators.BOX_ASSEMBLY
+
+
 def test_spmv_lanes(tmp_path):
     L = nat.lib()
     mesh = fa.TetrahedronMesh.from_box(nx=12, ny=12, nz=12, device=DEV)
