@@ -212,8 +212,9 @@ extern "C" int fa_element_vectors(int dtype, int td, int ldof, int nq, const dou
 extern "C" int fa_sep_sample(int td, int nq, const double* node, const int32_t* cell, int64_t nc, const void* sep,
                              double* out, fa_stream_t stream) {
     FA_REQUIRE(td == 2 || td == 3, "fa_sep_sample: td must be 2 or 3");
-    FA_REQUIRE(nq > 0 && nc >= 0 && sep && out, "fa_sep_sample: bad arguments");
-    if (nc == 0) return FA_OK;
+    FA_REQUIRE(nq > 0 && nc >= 0, "fa_sep_sample: bad sizes");
+    if (nc == 0) return FA_OK;  // an empty array may have no address
+    FA_REQUIRE(sep && out, "fa_sep_sample: bad arguments");
     const int cb = std::max(1, std::min(EV_CELLS, EV_POINTS / nq));
     const unsigned grid = grid_for(nc, cb, 256 * 8);
     const auto* se = static_cast<const fa_sep_t*>(sep);

@@ -1,6 +1,7 @@
 """Which kernel a call takes, where the rule can be asked without a device."""
 import pytest
 
+from fealpy_amd import _native as nat
 from fealpy_amd import expr
 from fealpy_amd.fem import integrators
 
@@ -20,3 +21,10 @@ def test_one_pass_load_vector_of_a_box(source, nq, n, one_pass):
 def test_separable_coefficient_sampled_first(points, ldof, sampled):
     """A launch more only where it gains: small P2 assemblies lost a tenth by it."""
     assert integrators._sampled_first(points, ldof) is sampled
+
+
+def test_sampling_no_cells_is_no_error():
+    """The element tensors of no cells are formed from arrays without an address, as in fa_element_matrices."""
+    L = nat.load()
+    assert L.fa_sep_sample(3, 4, None, None, 0, None, None, None) == nat.FA_OK
+    assert L.fa_sep_sample(3, 4, None, None, 1, None, None, None) == nat.FA_EINVAL
