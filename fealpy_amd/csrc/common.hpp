@@ -87,7 +87,6 @@ __device__ inline T wave_sum(T v) {
     return v;
 }
 
-// inclusive scan over a whole wavefront
 // XCD-aware workgroup order.  The dispatcher deals consecutive workgroups to
 // the 8 XCDs in turn, each with its own L2; renumbering workgroup b of a grid
 // of G (G a multiple of 8) as (b % 8) * (G / 8) + b / 8 gives every XCD one
@@ -115,6 +114,7 @@ __device__ inline unsigned xcd_window_block() {
 
 inline unsigned xcd_window_grid(unsigned g) { return (g + 8 * XCD_WINDOW - 1) / (8 * XCD_WINDOW) * (8 * XCD_WINDOW); }
 
+// inclusive scan over a whole wavefront
 __device__ inline int wave_inclusive_scan(int v) {
     const int lane = threadIdx.x & (WAVE - 1);
 #pragma unroll

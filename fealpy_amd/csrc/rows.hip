@@ -175,7 +175,7 @@ __global__ void __launch_bounds__(256) k_p1_rows(int64_t gdof, const int32_t* __
         incidence(k0);
         entries(h, p);
         incidence(k0 + 4);
-        for (int32_t k = k0; k < k1; k += 8) {  // two steps a turn, as above
+        for (int32_t k = k0; k < k1; k += 8) {  // two steps a turn: one's loads beside the other's adds
             entries(hn, pn);
             incidence(k + 8);
             add(k, h, p);
@@ -389,7 +389,7 @@ __global__ void __launch_bounds__(512) k_elasticity_rows(int64_t ns, int chunk, 
                         lds_add(o + x * drow + y * dcol, v);
                     }
             };
-            // two steps a turn, as in k_scalar_rows
+            // two steps a turn: the registers of one step are loaded while the other's are added
             for (int32_t k = 0; k < deg; k += 2) {
                 int q = p;
                 record(hn, in);
@@ -550,7 +550,9 @@ extern "C" int fa_vector_positions(int td, int dof_priority, int64_t ndof, int32
         return FA_ECAPACITY;
     }
     const unsigned grid = grid_for(ndof, waves, 1 << 20);
-#define FA_VP(TD_, PR_)                                                                                                hipLaunchKernelGGL((k_vector_positions<TD_, PR_>), dim3(grid), dim3(waves * WAVE), lds, S(stream), ndof, ldof,                        cell2dof, adj_ptr, adj, indptr, indices, lmax, pos)
+#define FA_VP(TD_, PR_)                                                                                          \
+    hipLaunchKernelGGL((k_vector_positions<TD_, PR_>), dim3(grid), dim3(waves * WAVE), lds, S(stream), ndof, ldof, \
+                       cell2dof, adj_ptr, adj, indptr, indices, lmax, pos)
     if (td == 2) {
         if (dof_priority) FA_VP(2, true);
         else FA_VP(2, false);
@@ -588,7 +590,14 @@ extern "C" int fa_assemble_elasticity_rows(int dtype, int td, int dof_priority, 
     else
         hipLaunchKernelGGL(k_elasticity_records<3>, dim3(rgrid), dim3(256), 0, s, nc, node_wide, cell, rec);
     FA_LAUNCH("k_elasticity_records");
-#define FA_CASE(TD_, L_)                                                                                                  if (td == TD_ && ldof == L_) {                                                                                            auto f = dof_priority ? (dtype == FA_F64 ? launch_elasticity_rows<TD_, L_, true, double>                                                                       : launch_elasticity_rows<TD_, L_, true, float>)                                                    : (dtype == FA_F64 ? launch_elasticity_rows<TD_, L_, false, double>                                                                      : launch_elasticity_rows<TD_, L_, false, float>);                            return f(ndof, nnz, table, cA, cB, cC, cD, adj_ptr, adj, indptr, pos, max_row, rec, values, s);                   }
+#define FA_CASE(TD_, L_)                                                                                         \
+    if (td == TD_ && ldof == L_) {                                                                               \
+        auto f = dof_priority ? (dtype == FA_F64 ? launch_elasticity_rows<TD_, L_, true, double>                 \
+                                                 : launch_elasticity_rows<TD_, L_, true, float>)                 \
+                              : (dtype == FA_F64 ? launch_elasticity_rows<TD_, L_, false, double>                \
+                                                 : launch_elasticity_rows<TD_, L_, false, float>);               \
+        return f(ndof, nnz, table, cA, cB, cC, cD, adj_ptr, adj, indptr, pos, max_row, rec, values, s);          \
+    }
     FA_CASE(2, 3) FA_CASE(2, 6) FA_CASE(2, 10) FA_CASE(2, 15) FA_CASE(3, 4) FA_CASE(3, 10) FA_CASE(3, 20)
 #undef FA_CASE
     set_error("fa_assemble_elasticity_rows: unsupported (td=%d, ldof=%d); p must be 1..4 (1..3 in 3D)", td, ldof);

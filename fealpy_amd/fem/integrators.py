@@ -411,6 +411,10 @@ def p1_matrix_values(space, ops, pat, dtype):
         spec[op] = coef_spec(it.coef, space, q, allow_sep=True)
     (dk, ds, dc), (mk, ms, mc) = spec['diff'], spec['mass']
     grid = _box_grid(space, pat)
+    if grid is None and pat.nc >= RECORDS_MIN_CELLS and max(dk, mk) <= nat.COEF_CELL:   # a record per cell, then the rows
+        v = p1_values(space, q, spec, pat, dtype)
+        if v is not None:
+            return v
     values = torch.empty(pat.nnz, dtype=dtype, device=space.device)
     if grid is not None:         # from_box tetrahedra: one pass, cells found from each node's grid position
         nat.check(L.fa_p1_box_matrix(nat.dtype_code(dtype), *grid, nat.ptr(mesh.node_rows16()),
@@ -418,10 +422,6 @@ def p1_matrix_values(space, ops, pat, dtype):
                                      nat.ptr(qw), nat.ptr(phi), dk, ds, nat.ptr(dc), mk, ms, nat.ptr(mc),
                                      nat.ptr(pat.indptr), pat.nnz, nat.ptr(values), nat.stream()), "fa_p1_box_matrix")
         return values
-    if pat.nc >= RECORDS_MIN_CELLS and max(dk, mk) <= nat.COEF_CELL:     # a record per cell, then the rows
-        v = p1_values(space, q, spec, pat, dtype)
-        if v is not None:
-            return v
     maps = pat.incidence_maps() if pat.nc >= TWO_PASS_MIN_CELLS else None
     if maps is not None:         # pass 1 per cell into incidence slots, pass 2 streams each row's slots
         # an FP32 matrix keeps its element rows in FP32 (half the slot traffic)
