@@ -57,7 +57,7 @@ def _reference(mesh, p, q, kd, km):
 
 
 SHAPES = [((1, 1), 1, 4), ((4, 8), 2, 5), ((3, 11), 3, 6), ((5, 7), 4, 9), ((2, 3), 2, 11), ((1, 1, 1), 1, 4),
-          ((2, 2, 3), 2, 5), ((3, 1, 4), 3, 5), ((2, 1, 3), 4, 6), ((1, 2, 1), 3, 9), ((2, 1, 1), 1, 9)]
+          ((2, 2, 3), 2, 5), ((3, 1, 4), 3, 5), ((2, 1, 3), 4, 6), ((1, 2, 3), 4, 7), ((1, 2, 1), 3, 9), ((2, 1, 1), 1, 9)]
 
 
 @pytest.mark.parametrize("dims,p,q", SHAPES)
@@ -131,3 +131,24 @@ def test_separable_coefficient_sampled_or_in_the_kernel(dims, p, monkeypatch):
         monkeypatch.setattr(integrators, "_sampled_first", lambda points, ldof: sampled)
         out.append(it.assembly(space))
     assert torch.equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("dims,p,q", [((15, 15, 15), 4, 7), ((30, 30, 30), 2, 11), ((260, 260), 2, 13)])
+@pytest.mark.parametrize("diff,mass", [("point", "point"), ("point", "cell")])
+def test_second_group_of_a_block(dims, p, q, diff, mass):
+    """More cells than one round of the capped grid, with rules of several chunks: a block stages the first points'
+    tables again for its next group.  The same cells alone, one group a block, have the same bits."""
+    mesh = _mesh(dims)
+    nc = mesh.number_of_cells()
+    nq = mesh.quadrature_formula(q).get_quadrature_points_and_weights()[1].shape[0]
+    assert nq > (56 if p == 4 else 64)
+    gen = torch.Generator(device=DEV).manual_seed(7)
+    kd = torch.rand((nc, nq), generator=gen, device=DEV, dtype=torch.float64) + 0.5
+    km = torch.rand((nc, nq) if mass == "point" else nc, generator=gen, device=DEV, dtype=torch.float64) + 0.5
+    idx = torch.arange(nc - 1, 0, -max(nc // 500, 1), device=DEV)
+
+    def elements(a, b, indices):
+        return fa.GroupIntegrator(fa.ScalarDiffusionIntegrator(a, q=q), fa.ScalarMassIntegrator(b, q=q)).assembly(
+            fa.LagrangeFESpace(mesh, p), indices=indices)
+
+    assert torch.equal(elements(kd, km, None)[idx], elements(kd[idx].contiguous(), km[idx].contiguous(), idx))

@@ -39,6 +39,7 @@ def _fan(n):
 MESHES = {"tri1": lambda: fa.TriangleMesh.from_box(nx=1, ny=1, device=DEV),
           "tri": lambda: _shuffled(fa.TriangleMesh.from_box(nx=9, ny=7, device=DEV), 1),
           "fan": lambda: _fan(300),
+         "fan100": lambda: _fan(100),
           "tet1": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=1, ny=1, nz=1, device=DEV), 2),
           "tet2": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=2, ny=1, nz=2, device=DEV), 5),
          "tet": lambda: _shuffled(fa.TetrahedronMesh.from_box(nx=4, ny=3, nz=5, device=DEV), 3)}
@@ -64,13 +65,16 @@ def _check(A, space, elem, dtype):
 @pytest.mark.parametrize("ops", ["diff", "mass", "both"])
 def test_p1_rows(name, dtype, ops, monkeypatch):
     monkeypatch.setattr(integrators, "RECORDS_MIN_CELLS", 0)
-    mesh = MESHES[name]()
+    mesh, calls = MESHES[name](), []
+    monkeypatch.setattr(integrators, "p1_values", lambda *a: calls.append(rows.p1_values(*a)) or calls[-1])
     space = fa.LagrangeFESpace(mesh, 1)
     k = torch.as_tensor(np.exp(np.random.default_rng(4).standard_normal(mesh.number_of_cells())), device=DEV)
     ints = [fa.ScalarDiffusionIntegrator(k, q=3)] if ops != "mass" else []
     ints += [fa.ScalarMassIntegrator(0.5 if ops == "both" else k, q=3)] if ops != "diff" else []
     group = fa.GroupIntegrator(*ints)
     A = fa.BilinearForm(space).add_integrator(group).assembly(dtype=dtype)
+    # rows of more than 128 entries are summed from element matrices
+    assert [v is not None for v in calls] == ([] if name == "fan" else [True])
     _check(A, space, group.assembly(space), dtype)
 
 
