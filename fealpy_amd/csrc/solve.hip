@@ -111,7 +111,9 @@ __global__ void __launch_bounds__(256) k_spmm(int64_t n, int64_t nv, const int32
 }
 
 // lanes per row: so many that a block's 256 / G rows hold one to two
-// thousand entries on average
+// thousand entries on average.  Against 4 lanes and more a row, each row read by
+// its own (1000^2 P1 33.6 -> 21 us, 400^2 P2 34 -> 26, 60^3 P1 14.1 -> 10.2, 128^3
+// 149 -> 84); matrices of a few blocks (20^2 to 300^2) take a launch either way
 static int lanes_for(int64_t n, int64_t nnz) {
     const double avg = n > 0 ? double(nnz) / double(n) : 1.0;
     int g = 1;
@@ -261,7 +263,11 @@ template <class T, class U, int VAL, bool RHS>
 static int bc_launch(int64_t n, const int32_t* indptr, const int32_t* indices, const void* vals, const uint8_t* bd,
                      const int32_t* nptr, int32_t* nidx, void* nval, const void* uh, const void* f, void* out,
                      hipStream_t s) {
-    constexpr int G = 4;  // 64 rows a block: 960 entries of a P1 tetrahedral matrix, a chunk
+    // 64 rows a block: 960 entries of a P1 tetrahedral matrix, a chunk; also faster
+    // than 16 lanes a row where a block fills half a chunk or takes two (whole
+    // boundary condition, 1000^2 P1 127 -> 72 us, 400^2 P2 98 -> 64, 40^3 P2
+    // 123 -> 91; at 300^2 and below the launches take it all)
+    constexpr int G = 4;
     hipLaunchKernelGGL((k_bc_rows<T, U, G, VAL, RHS>), dim3(xcd_window_grid(grid_for(n * G, 256, 1 << 20))), dim3(256), 0, s,
                        n, indptr, indices, static_cast<const T*>(vals), bd, nptr, nidx, static_cast<U*>(nval),
                        static_cast<const T*>(uh), static_cast<const T*>(f), static_cast<T*>(out));
